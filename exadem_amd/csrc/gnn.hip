@@ -8,9 +8,8 @@
 //   out = h W_out^T + b_out
 // Dense products over particles (P|Q, U and their backward and weight-gradient products) run on
 // MFMA (v_mfma_f32_32x32x16_bf16); the per-edge work (messages and their backward) is a segment sum
-// over each particle's list entries, one wavefront per particle, two channels per lane. The backward
-// of the Q side reads the reverse entry of every edge (its mirror slot), so no atomics are used and
-// every reduction has a fixed order.
+// over each particle's list entries, also on MFMA. The backward of the Q side reads the reverse entry of
+// every edge (its mirror slot), so no atomics are used and every reduction has a fixed order.
 //
 // HBM layout per network: node inputs x [n][8] bf16, edge inputs e [slots][16] bf16 (same slot index
 // as the neighbour list), hidden h [n][128] bf16 (L+1 copies when training), P|Q [n][256] bf16,
@@ -485,26 +484,12 @@ struct MsgArgs {
   uint16_t* m;       // forward output [n][H]
   const float* dm;   // backward input [n][H]
   const uint32_t* mirror;
+  uint32_t* gate;    // [slots][H / 32]: bit c % 32 of word c / 32 is set where z_ij > 0 in channel c
   uint16_t* dpq;     // backward output [n][2H]
   float* part_w;     // backward partials [blocks][H][FE]
   float* part_b;     // [blocks][H]
 };
 
-__device__ inline void load_e(const uint16_t* p, float ev[FE]) {
-  uint4 pk[2];
-  pk[0] = ((const uint4*)p)[0];
-  pk[1] = ((const uint4*)p)[1];
-  uint16_t t[FE];
-  memcpy(t, pk, 32);
-#pragma unroll
-  for (int k = 0; k < FE; k++) ev[k] = bf2f(t[k]);
-}
-__device__ inline float edge_z(float P, float Q, const float ev[FE], const float w[FE], float b) {
-  float E = 0.f;
-#pragma unroll
-  for (int k = 0; k < FE; k++) E = fmaf(w[k], ev[k], E);
-  return ((P + Q) + E) + b;
-}
 __device__ inline void ld2(const uint16_t* p, float& a, float& b) {
   const uint32_t v = *(const uint32_t*)p;
   a = bf2f((uint16_t)(v & 0xffffu));
@@ -620,77 +605,219 @@ __global__ __launch_bounds__(256) void k_msg_fwd_mfma(MsgArgs a, const uint16_t*
   *(uint4*)(a.m + i * H + c0 + 8) = uint4{o[4], o[5], o[6], o[7]};
 }
 
-// backward of the messages: per particle j, dP_j = sum over own entries j->i of dm_j (z_ji > 0),
-// dQ_j = sum over the reverse entries i->j of dm_i (z_ij > 0); W_E and b_E gradients over own entries
-__global__ __launch_bounds__(256) void k_msg_bwd(MsgArgs a) {
-  __shared__ float red[4][H * (FE + 1)];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int c = 2 * lane;
-  float w0[FE], w1[FE];
-#pragma unroll
-  for (int k = 0; k < FE; k++) {
-    w0[k] = a.wE[c * FE + k];
-    w1[k] = a.wE[(c + 1) * FE + k];
+// Backward of the messages over each particle's own entries, on MFMA: z is formed again as in the forward pass,
+// but with the edges as MFMA rows and the channels as columns, because every product that follows needs a lane
+// to hold one channel of many edges: accumulator element v of lane l is edge row 8(v/4) + 4(l/32) + v%4 of
+// channel l%32 of the wavefront's 32. One block of four wavefronts per 32 consecutive particles i (half of a list
+// group) at a time, 32 channels per wavefront; step k takes list rank k of each particle, so a row is the same
+// particle in every step and dP_i = sum_k [z_ik > 0] dm_i is summed in the accumulator layout. A padding slot's
+// Q row is -3e38 in every channel, which closes its gate.
+//
+// gW_E[f][c] = sum over edges of e[f] g[c] with g = [z > 0] dm is one more product, over the edges: its B operand
+// (8 edges of one channel per lane and k step) is exactly the lane's accumulator elements 8s .. 8s+7, the A
+// operand the same edges' inputs, read back transposed from the wavefront's LDS copy, with row 16 = 1 for the
+// bias. dm keeps its 32 bits: it enters as the exact sum of three bfloat16 parts, split once per particle group,
+// whose halves the gates then mask.
+//
+// The gates go to `gate` (128 bits per slot), so that the partner's side (k_msg_bwd_q) need not form z again.
+// Replaces one wavefront per particle with two channels per lane, which spent 250 vector instructions per edge
+// and one dependent chain of gathers per edge: 592 us per layer at 50k spheres (297k entries), now 45 us with
+// k_msg_bwd_q.
+struct BwdStep {
+  bool ok;
+  uint4 e;
+  uint4 q[2];
+};
+__device__ inline void bwd_load(const MsgArgs& a, uint64_t sl, bool ok, uint32_t wd, int half, int ch0, BwdStep& st) {
+  st.ok = ok;
+  if (ok) {
+    st.e = *(const uint4*)(a.e + sl * FE + 8 * half);
+    const uint16_t* qrow = a.pq + (int64_t)(wd & kIdxMask) * H2 + H + ch0 + 8 * half;
+    st.q[0] = *(const uint4*)(qrow);
+    st.q[1] = *(const uint4*)(qrow + 16);
+  } else {
+    st.e = uint4{0u, 0u, 0u, 0u};
+    st.q[0] = st.q[1] = uint4{0xff61ff61u, 0xff61ff61u, 0xff61ff61u, 0xff61ff61u};  // -3e38, finite
   }
-  const float b0 = a.bE[c], b1 = a.bE[c + 1];
-  float gw0[FE], gw1[FE], gb0 = 0.f, gb1 = 0.f;
+}
+// v_writelane_b32: `old` with its value in one lane replaced by the uniform `val` (no clang builtin; the compiler's
+// own intrinsic, so that it keeps the instruction's hazards)
+__device__ int amdgcn_writelane(int val, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ inline uint32_t write_lane(uint32_t old, uint32_t val, int lane) {
+  return (uint32_t)amdgcn_writelane((int)val, lane, (int)old);
+}
+// orders this wavefront's LDS accesses across its lanes (nothing is executed)
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ inline bf16x8 as_frag(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+constexpr int kBwdERow = 24;  // LDS row of an edge's 16 inputs: 48 bytes (16-byte aligned, rows spread over banks)
+__global__ __launch_bounds__(256) void k_msg_bwd(MsgArgs a, const uint16_t* __restrict__ wEb, int ngroups) {
+  __shared__ uint16_t et[4][32 * kBwdERow];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int ch0 = w * 32;
+  uint16_t* ew = et[w];
+  const bf16x8 wb = *(const bf16x8*)(wEb + (ch0 + col) * FE + 8 * half);
+  // identity columns: input channel 8 half + q (and 16 more) to column `col`
+  uint32_t ia[4], ib[4];
 #pragma unroll
-  for (int k = 0; k < FE; k++) gw0[k] = gw1[k] = 0.f;
-  const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
-  for (int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; j < a.n; j += nw) {
-    float Pj0, Pj1, Qj0, Qj1;
-    ld2(a.pq + j * H2 + c, Pj0, Pj1);
-    ld2(a.pq + j * H2 + H + c, Qj0, Qj1);
-    const float dmj0 = a.dm[j * H + c], dmj1 = a.dm[j * H + c + 1];
-    const uint32_t cnt = a.nl.cnt[j];
-    const uint64_t base = a.nl.base[j >> 6] + (uint64_t)(j & 63);
-    float dP0 = 0.f, dP1 = 0.f, dQ0 = 0.f, dQ1 = 0.f;
-    for (uint32_t k = 0; k < cnt; k++) {
-      const uint64_t sl = base + (uint64_t)k * kWave;
-      const uint32_t i = a.nl.word[sl] & kIdxMask;
-      float Pi0, Pi1, Qi0, Qi1;
-      ld2(a.pq + (int64_t)i * H2 + c, Pi0, Pi1);
-      ld2(a.pq + (int64_t)i * H2 + H + c, Qi0, Qi1);
-      // own entry j -> i
-      float ev[FE];
-      load_e(a.e + sl * FE, ev);
-      const float g0 = edge_z(Pj0, Qi0, ev, w0, b0) > 0.f ? dmj0 : 0.f;
-      const float g1 = edge_z(Pj1, Qi1, ev, w1, b1) > 0.f ? dmj1 : 0.f;
-      dP0 += g0;
-      dP1 += g1;
-      gb0 += g0;
-      gb1 += g1;
+  for (int q = 0; q < 4; q++) {
+    const int k0 = 8 * half + 2 * q;
+    ia[q] = (col == k0 ? 0x3f80u : 0u) | (col == k0 + 1 ? 0x3f800000u : 0u);
+    ib[q] = (col == 16 + k0 ? 0x3f80u : 0u) | (col == 16 + k0 + 1 ? 0x3f800000u : 0u);
+  }
+  const bf16x8 id0 = as_frag(uint4{ia[0], ia[1], ia[2], ia[3]}), id1 = as_frag(uint4{ib[0], ib[1], ib[2], ib[3]});
+  const float bias = a.bE[ch0 + col];
+  floatx16 gw;
 #pragma unroll
-      for (int q = 0; q < FE; q++) {
-        gw0[q] = fmaf(g0, ev[q], gw0[q]);
-        gw1[q] = fmaf(g1, ev[q], gw1[q]);
-      }
-      // reverse entry i -> j
-      const uint64_t ms = a.mirror[sl];
-      float er[FE];
-      load_e(a.e + ms * FE, er);
-      const float dmi0 = a.dm[(int64_t)i * H + c], dmi1 = a.dm[(int64_t)i * H + c + 1];
-      dQ0 += edge_z(Pi0, Qj0, er, w0, b0) > 0.f ? dmi0 : 0.f;
-      dQ1 += edge_z(Pi1, Qj1, er, w1, b1) > 0.f ? dmi1 : 0.f;
+  for (int v = 0; v < 16; v++) gw[v] = 0.f;
+  for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
+    const int64_t i0 = (int64_t)grp * 32;
+    const int64_t i = i0 + col;
+    const bool vi = i < a.n;
+    const int64_t ic = vi ? i : a.n - 1;
+    const uint64_t base = a.nl.base[i0 >> 6] + (uint64_t)(ic & 63);
+    const uint32_t cnt = vi ? a.nl.cnt[ic] : 0u;
+    const uint32_t kmax = a.nl.kmax[i0 >> 6];
+    BwdStep cur, nxt;
+    uint32_t wnext = 0;
+    uint64_t slc = base;
+    if (kmax > 0) {
+      bwd_load(a, base, cnt > 0, cnt > 0 ? a.nl.word[base] : 0u, half, ch0, cur);
+      if (cnt > 1) wnext = a.nl.word[base + kWave];
     }
-    *(uint32_t*)(a.dpq + j * H2 + c) = pack_bf16(dP0, dP1);
-    *(uint32_t*)(a.dpq + j * H2 + H + c) = pack_bf16(dQ0, dQ1);
-  }
-  // block reduction of the W_E / b_E gradients in wavefront order
+    // P_i + b_E in the accumulator layout, and dm of the lane's 16 rows with its three bfloat16 parts
+    const uint16_t* prow = a.pq + ic * H2 + ch0 + 8 * half;
+    floatx16 zp;
 #pragma unroll
-  for (int k = 0; k < FE; k++) {
-    red[wv][c * (FE + 1) + k] = gw0[k];
-    red[wv][(c + 1) * (FE + 1) + k] = gw1[k];
+    for (int v = 0; v < 16; v++) zp[v] = bias;
+    zp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)prow, id0, zp, 0, 0, 0);
+    zp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(prow + 16), id1, zp, 0, 0, 0);
+    float dmv[16], dp[16];
+    uint32_t d1[8], d2[8], d3[8];
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int64_t p = i0 + 8 * (v >> 2) + 4 * half + (v & 3);
+      dmv[v] = p < a.n ? a.dm[p * H + ch0 + col] : 0.f;
+      dp[v] = 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      float r0 = dmv[2 * t], r1 = dmv[2 * t + 1];
+      d1[t] = pack_bf16(r0, r1);
+      r0 -= bf_lo(d1[t]);
+      r1 -= bf_hi(d1[t]);
+      d2[t] = pack_bf16(r0, r1);
+      r0 -= bf_lo(d2[t]);
+      r1 -= bf_hi(d2[t]);
+      d3[t] = pack_bf16(r0, r1);
+    }
+    for (uint32_t k = 0; k < kmax; k++) {
+      if (k + 1 < kmax) {
+        const uint64_t sl1 = base + (uint64_t)(k + 1) * kWave;
+        bwd_load(a, sl1, k + 1 < cnt, wnext, half, ch0, nxt);
+        wnext = k + 2 < cnt ? a.nl.word[sl1 + kWave] : 0u;
+      }
+      floatx16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(cur.e), wb, zp, 0, 0, 0);
+      z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(cur.q[0]), id0, z, 0, 0, 0);
+      z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(cur.q[1]), id1, z, 0, 0, 0);
+      // the copy is the wavefront's own: its lanes' LDS accesses stay in program order
+      wave_fence();
+      *(uint4*)(ew + col * kBwdERow + 8 * half) = cur.e;
+      wave_fence();
+      uint32_t gword = 0;
+      uint32_t keep[8];
+#pragma unroll
+      for (int t = 0; t < 8; t++) keep[t] = 0u;
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const bool on = z[v] > 0.f;
+        dp[v] += on ? dmv[v] : 0.f;
+        keep[v >> 1] |= on ? ((v & 1) ? 0xffff0000u : 0xffffu) : 0u;
+        // the gate words of edge rows 8(v/4) + v%4 (low half of the ballot) and + 4 (high half)
+        const uint64_t bal = __builtin_amdgcn_ballot_w64(on);
+        const int row = 8 * (v >> 2) + (v & 3);
+        gword = write_lane(gword, (uint32_t)bal, row);
+        gword = write_lane(gword, (uint32_t)(bal >> 32), row + 4);
+      }
+      if (half == 0 && cur.ok) a.gate[slc * 4 + w] = gword;
+      // e transposed: row f = col (16 inputs, then the constant 1), the 8 edges of k step s
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        uint32_t ef[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const int r = 16 * s + 8 * (t >> 1) + 4 * half + 2 * (t & 1);
+          const uint32_t lo = ew[r * kBwdERow + (col & 15)], hi = ew[(r + 1) * kBwdERow + (col & 15)];
+          ef[t] = col < FE ? (lo | (hi << 16)) : (col == FE ? 0x3f803f80u : 0u);
+        }
+        const bf16x8 ea = as_frag(uint4{ef[0], ef[1], ef[2], ef[3]});
+        const uint32_t* kp = keep + 4 * s;
+        const uint32_t *p1 = d1 + 4 * s, *p2 = d2 + 4 * s, *p3 = d3 + 4 * s;
+        gw = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            ea, as_frag(uint4{p1[0] & kp[0], p1[1] & kp[1], p1[2] & kp[2], p1[3] & kp[3]}), gw, 0, 0, 0);
+        gw = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            ea, as_frag(uint4{p2[0] & kp[0], p2[1] & kp[1], p2[2] & kp[2], p2[3] & kp[3]}), gw, 0, 0, 0);
+        gw = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            ea, as_frag(uint4{p3[0] & kp[0], p3[1] & kp[1], p3[2] & kp[2], p3[3] & kp[3]}), gw, 0, 0, 0);
+      }
+      cur = nxt;
+      slc += kWave;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int64_t p = i0 + 8 * (v >> 2) + 4 * half + (v & 3);
+      if (p < a.n) a.dpq[p * H2 + ch0 + col] = f2bf(dp[v]);
+    }
   }
-  red[wv][c * (FE + 1) + FE] = gb0;
-  red[wv][(c + 1) * (FE + 1) + FE] = gb1;
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < H * (FE + 1); idx += blockDim.x) {
-    const float s = ((red[0][idx] + red[1][idx]) + red[2][idx]) + red[3][idx];
-    const int ch = idx / (FE + 1), k = idx % (FE + 1);
-    if (k < FE) a.part_w[(int64_t)blockIdx.x * H * FE + ch * FE + k] = s;
-    else a.part_b[(int64_t)blockIdx.x * H + ch] = s;
+  // rows 0..15 of gw are the inputs, row 16 (element 8 of half 0) the bias
+#pragma unroll
+  for (int v = 0; v < 8; v++)
+    a.part_w[(int64_t)blockIdx.x * H * FE + (ch0 + col) * FE + 8 * (v >> 2) + 4 * half + (v & 3)] = gw[v];
+  if (half == 0) a.part_b[(int64_t)blockIdx.x * H + ch0 + col] = gw[8];
+}
+
+// The partner's side: dQ_j = sum over j's entries of dm_i where the reverse entry i -> j (its mirror slot) has its
+// gate open, in list order. One wavefront per particle, two channels per lane; the entries' words and mirror slots
+// are read by one lane each and handed round as scalars, and eight entries' rows are in flight at a time.
+__global__ __launch_bounds__(256) void k_msg_bwd_q(MsgArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t j = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
+  if (j >= a.n) return;
+  const uint32_t cnt = a.nl.cnt[j];
+  const uint64_t base = a.nl.base[j >> 6] + (uint64_t)(j & 63);
+  const int c = 2 * lane;
+  float dq0 = 0.f, dq1 = 0.f;
+  for (uint32_t k0 = 0; k0 < cnt; k0 += 64) {
+    const uint32_t m = cnt - k0 < 64u ? cnt - k0 : 64u;
+    uint32_t wd = 0, ms = 0;
+    if ((uint32_t)lane < m) {
+      const uint64_t sl = base + (uint64_t)(k0 + lane) * kWave;
+      wd = a.nl.word[sl] & kIdxMask;
+      ms = a.mirror[sl];
+    }
+    for (uint32_t k = 0; k < m; k += 8) {
+      uint32_t g[8];
+      float2v d[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const uint32_t kq = k + q < m ? k + q : k;  // past the end: the batch's first entry again, not added
+        const uint32_t i = __builtin_amdgcn_readlane((int)wd, (int)kq), s = __builtin_amdgcn_readlane((int)ms, (int)kq);
+        g[q] = a.gate[(uint64_t)s * 4 + (lane >> 4)];
+        d[q] = *(const float2v*)(a.dm + (int64_t)i * H + c);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const uint32_t bits = k + q < m ? g[q] >> (c & 31) : 0u;
+        dq0 += (bits & 1u) ? d[q].x : 0.f;
+        dq1 += (bits & 2u) ? d[q].y : 0.f;
+      }
+    }
   }
+  *(uint32_t*)(a.dpq + j * H2 + H + c) = pack_bf16(dq0, dq1);
 }
 
 // ------------------------------------------------------------------------------------- decoder
@@ -1079,6 +1206,7 @@ struct xdem_gnn {
   uint16_t* du = nullptr;
   uint16_t* dpq = nullptr;
   uint32_t* mirror = nullptr;
+  uint32_t* gate = nullptr;  // gates of the messages' backward pass (MsgArgs::gate)
   float* partial = nullptr;  // partial sums of the reductions (sized once, never reallocated)
   int64_t cap_partial = 0;
   float* dec_sum = nullptr;  // decoder reduction: dW_out, db_out, loss
@@ -1110,7 +1238,7 @@ int ensure_buffers(xdem_gnn* G) {
   if (nl.slots > G->cap_slots) {
     const int64_t cap = (int64_t)(nl.slots * 1.25) + 4096;
     if ((rc = galloc(c, &G->e, cap * FE))) return rc;
-    if (G->cfg.train && (rc = galloc(c, &G->mirror, cap))) return rc;
+    if (G->cfg.train && ((rc = galloc(c, &G->mirror, cap)) || (rc = galloc(c, &G->gate, cap * (H / 32))))) return rc;
     G->cap_slots = cap;
   }
   if (n > G->cap_n) {
@@ -1308,14 +1436,15 @@ int backward(xdem_gnn* G, double* loss) {
     g1.m = H2; g1.dh = G->dh; g1.dm = G->dm;
     if ((rc = gemm_p<EPI_BWD_U, H2, H, 0>(G, g1))) return rc;
     // messages: dP|dQ, dW_E, db_E
-    const int mb = wgrid;
+    const int ngroups = nb(n, 32), mb = std::min(ngroups, kRedBlocks);
     if ((rc = ensure_partial(G, (int64_t)mb * H * (FE + 1)))) return rc;
     MsgArgs ma{};
     ma.n = n; ma.nl = nl; ma.e = G->e; ma.pq = G->pq[l];
     ma.wE = G->wr + G->off.W_E[l]; ma.bE = G->wr + G->off.b_E[l];
-    ma.dm = G->dm; ma.mirror = G->mirror; ma.dpq = G->dpq;
+    ma.dm = G->dm; ma.mirror = G->mirror; ma.gate = G->gate; ma.dpq = G->dpq;
     ma.part_w = G->partial; ma.part_b = G->partial + (int64_t)mb * H * FE;
-    hipLaunchKernelGGL(k_msg_bwd, dim3(mb), dim3(256), 0, c->stream, ma);
+    hipLaunchKernelGGL(k_msg_bwd, dim3(mb), dim3(256), 0, c->stream, ma, G->wbf + G->off.W_E[l], ngroups);
+    hipLaunchKernelGGL(k_msg_bwd_q, dim3(nb(n, 4)), dim3(256), 0, c->stream, ma);
     hipLaunchKernelGGL(k_sum_partials, dim3(nb((int64_t)H * FE, 256)), dim3(256), 0, c->stream, ma.part_w, mb,
                        (int64_t)H * FE, G->g + G->off.W_E[l]);
     hipLaunchKernelGGL(k_sum_partials, dim3(nb(H, 256)), dim3(256), 0, c->stream, ma.part_b, mb, (int64_t)H,
@@ -1387,7 +1516,7 @@ extern "C" int xdem_gnn_destroy(xdem_gnn* G) {
   (void)hipStreamSynchronize(G->c->stream);
   void* bufs[] = {G->p,  G->g,   G->m1,     G->m2,      G->wbf,     G->wr,      G->wT,
                   G->x,  G->e,   G->out,    G->target,  G->dh,      G->dm,      G->du,
-                  G->dpq, G->mirror, G->partial, G->snap, G->xs, G->xf, G->dpart, G->dec_sum};
+                  G->dpq, G->mirror, G->gate, G->partial, G->snap, G->xs, G->xf, G->dpart, G->dec_sum};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (int k = 0; k <= L; k++)

@@ -127,6 +127,44 @@ def test_backward_matches_oracle(net):
         assert np.linalg.norm(a - b) <= 2e-2 * nb_, (name, np.linalg.norm(a - b) / nb_)
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 257, 1025])
+def test_backward_sizes_match_oracle(gpu_ok, n):
+    """Gradients at the edges of the kernels' tiles (32 particles, 64-particle list groups, 256-row strips), on
+    walled lattices with overlaps; n = 1 has no list entry. The bar is the bfloat16 one of the larger test: two
+    bfloat16 pipelines that round at the same points differ by about 2^-9 per stored value, 2e-2 leaves room
+    for the gates that such a difference flips."""
+    from exadem_amd import inputs
+    side = max(4, int(np.ceil((n / 1.5) ** (1.0 / 3.0))))
+    edge = 0.98 * (side - 1) + 0.96
+    w = inputs.deposition(n=n, spacing=0.98, seed=n, start=0.48, box=(edge, edge, 2 * edge + 2))
+    rng = np.random.default_rng(n)
+    for k in ("vx", "vy", "vz", "vrotx", "vroty", "vrotz"):
+        w.particles[k] = rng.normal(0, 0.1, n)
+    sim = SphereSim(w)
+    sim.first_iteration()
+    flat = _params(n + 4)
+    gnn = native.Gnn(sim.ctx, r0=0.4, v0=0.1, a0=1.0, m0=4000.0, ov_scale=50.0, substeps=10, train=True)
+    gnn.set_params(flat)
+    out = gnn.forward()
+    target = (out + rng.normal(0, 0.5, out.shape)).astype(np.float32)
+    gnn.set_target(target)
+    loss = gnn.backward()
+    grads = gnn.get_grads()
+    src, dst, e, x = gnn.dump_graph()
+    onet = G.Net(flat.astype(np.float64), exact=False)
+    o_out, cache = onet.forward(x, src.astype(np.int64), dst.astype(np.int64), e)
+    assert loss == pytest.approx(onet.loss(o_out, target), rel=2e-2)
+    og = onet.backward(cache, target)
+    off = 0
+    for name, shape in G.param_layout():
+        k = int(np.prod(shape))
+        a, b = grads[off:off + k].astype(np.float64), np.asarray(og[name], np.float64).ravel()
+        off += k
+        nb_ = np.linalg.norm(b)
+        assert np.linalg.norm(a - b) <= 2e-2 * nb_ + 1e-12, (name, np.linalg.norm(a - b), nb_)
+    gnn.close()
+
+
 def test_training_lowers_loss_and_beats_free_flight(gpu_ok):
     """The library's training loop on 16 packings of 4000 spheres (25 windows of 10 DEM steps each);
     then, on windows of a packing it has not seen, the network's acceleration error against the DEM
