@@ -26,8 +26,11 @@ namespace gnn {
 constexpr int H = XDEM_GNN_HIDDEN, L = XDEM_GNN_LAYERS, FN = 8, FE = 16, FO = 6, H2 = 2 * H;
 constexpr float kMsgScale = 0.125f;
 constexpr int kRedBlocks = 512;  // blocks of the grid-stride reduction kernels (partial sums)
-// largest partial-sum need: 256 weight-gradient blocks of 128 x 256 floats
-constexpr int64_t kPartialFloats = (int64_t)256 * 128 * 256 + 65536;
+constexpr int kWgChunks = 128;   // most row chunks of a weight gradient
+// partial sums of one backward pass: per layer two weight gradients of H x 2H with a bias and the message
+// gradients, then the decoder (its outputs and the loss) and the encoder
+constexpr int64_t kPartialFloats = (int64_t)L * (kWgChunks * (2 * H * H2 + H) + kRedBlocks * H * (FE + 1)) +
+                                   (int64_t)kRedBlocks * (FO * H + FO + 1 + H * (FN + 1));
 
 struct Off {
   int64_t W_in, b_in, W_AB[L], W_E[L], b_E[L], W_U[L], b_U[L], W_out, b_out, total;
@@ -376,101 +379,147 @@ __global__ __launch_bounds__(512) void k_gemm_p(GemmArgs g) {
   }
 }
 
-// Weight gradient Gw[m][k] = sum_r G[r][m] X[r][k] (G [n][mg], X = [x1 | x2] [n][k1+k2], all bf16):
-// each block reduces a contiguous range of rows in steps of 16 (the MFMA k dimension), staging the
-// 16 rows of G and X in LDS, and writes its mg x K partial sum; k_sum_partials adds the partials.
-// mg * K = 32768: 32 tiles of 32x32, 8 per wavefront.
+// Weight gradient Gw[m][k] = sum_r G[r][m] X[r][k] (G, X bf16, r over particles) and, where asked for, the bias
+// gradient sum_r G[r][m]. The contraction runs over rows, so both operands are wanted with consecutive rows in a
+// lane: a block stages 64 rows of 128 columns of G and of X in LDS transposed (a thread loads 8 rows x 8 columns,
+// transposes them in registers with byte permutes and writes 16 bytes per column; column stride 144 bytes, so
+// writes and reads fall on distinct banks), with the next 64 rows' loads in flight meanwhile. Four wavefronts form
+// 64 x 64 each of the 128 x 128 output. The two halves of the 32,768 outputs go to two sets of blocks (blockIdx.y),
+// the rows to blockIdx.x; the partial sums are added by k_reduce in a fixed order. The bias is the product with a
+// column of ones. Reading the operands element by element from row-major tiles, in blocks of all 32,768 outputs,
+// took 53 us per gradient at 50k rows and 24 us for the bias in a pass of its own; now 16 us with the bias.
+struct WgradHalf {
+  const uint16_t* g;  // first of 128 columns of G
+  const uint16_t* x;  // first of 128 columns of X
+  int ldg, ldx;
+  int64_t out;  // offset of the half in the [mg][K] output
+};
 struct WgradArgs {
   int64_t n;
-  const uint16_t* gm;
-  int mg;
-  const uint16_t* x1;
-  int k1;
-  const uint16_t* x2;
-  int k2;
+  WgradHalf h[2];
+  int ldo;
   int64_t rows_per_block;
-  float* partial;  // [gridDim.x][mg][K]
+  float* partial;  // [gridDim.x][mg * K]
+  float* part_b;   // [gridDim.x][128] (null: no bias gradient)
 };
+constexpr int kWgRows = 64, kWgStride = kWgRows + 8;
 __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
-  __shared__ uint16_t sg[16 * 256];
-  __shared__ uint16_t sx[16 * 256];
+  __shared__ uint16_t tile[256 * kWgStride];
+  const WgradHalf hf = a.h[blockIdx.y];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int K = a.k1 + a.k2;
-  const int tk = K / 32;
-  floatx16 acc[8];
+  const int col = lane & 31, half = lane >> 5;
+  const int m0 = (w & 1) * 64, k0 = (w >> 1) * 64;
+  const bool bias = a.part_b && blockIdx.y == 0 && k0 == 0;
+  floatx16 acc[2][2], accb[2];
 #pragma unroll
-  for (int t = 0; t < 8; t++)
-    for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[i][0][v] = acc[i][1][v] = accb[i][v] = 0.f;
   const int64_t rbeg = (int64_t)blockIdx.x * a.rows_per_block;
   const int64_t rend = std::min<int64_t>(a.n, rbeg + a.rows_per_block);
-  for (int64_t r0 = rbeg; r0 < rend; r0 += 16) {
-    __syncthreads();
-    // stage 16 rows: G row-major [16][mg], X [16][K]; zero beyond the range
-    for (int idx = threadIdx.x; idx < 16 * a.mg / 8; idx += 256) {
-      const int rr = idx / (a.mg / 8), cc = (idx % (a.mg / 8)) * 8;
-      uint4 v = {0, 0, 0, 0};
-      if (r0 + rr < rend) v = *(const uint4*)(a.gm + (r0 + rr) * a.mg + cc);
-      *(uint4*)(sg + rr * a.mg + cc) = v;
-    }
-    for (int idx = threadIdx.x; idx < 16 * K / 8; idx += 256) {
-      const int rr = idx / (K / 8), cc = (idx % (K / 8)) * 8;
-      uint4 v = {0, 0, 0, 0};
-      if (r0 + rr < rend) {
-        if (cc < a.k1) v = *(const uint4*)(a.x1 + (r0 + rr) * a.k1 + cc);
-        else v = *(const uint4*)(a.x2 + (r0 + rr) * a.k2 + (cc - a.k1));
-      }
-      *(uint4*)(sx + rr * K + cc) = v;
-    }
-    __syncthreads();
-    const int rk = 8 * (lane >> 5);
+  // this thread's 8 rows x 8 columns of each stage
+  const int rb = threadIdx.x & 7, cb = threadIdx.x >> 3;
+  const bool isg = cb < 16;
+  const uint16_t* src = isg ? hf.g + 8 * cb : hf.x + 8 * (cb - 16);
+  const int ld = isg ? hf.ldg : hf.ldx;
+  uint4 in[8];
+  auto load = [&](int64_t r0) {
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      const int tile = w * 8 + t;
-      const int ti = tile / tk, tj = tile % tk;
-      const int mrow = ti * 32 + (lane & 31), kcol = tj * 32 + (lane & 31);
-      bf16x8 av, bv;
-      uint16_t ta[8], tb[8];
+    for (int q = 0; q < 8; q++) {
+      const int64_t r = r0 + 8 * rb + q;
+      in[q] = r < rend ? *(const uint4*)(src + r * ld) : uint4{0u, 0u, 0u, 0u};
+    }
+  };
+  if (rbeg < rend) load(rbeg);
+  for (int64_t r0 = rbeg; r0 < rend; r0 += kWgRows) {
+    uint32_t o[8][4];
 #pragma unroll
-      for (int s = 0; s < 8; s++) {
-        ta[s] = sg[(rk + s) * a.mg + mrow];
-        tb[s] = sx[(rk + s) * K + kcol];
+    for (int p = 0; p < 4; p++) {
+      const uint32_t x[4] = {in[2 * p].x, in[2 * p].y, in[2 * p].z, in[2 * p].w};
+      const uint32_t y[4] = {in[2 * p + 1].x, in[2 * p + 1].y, in[2 * p + 1].z, in[2 * p + 1].w};
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        o[2 * c][p] = __builtin_amdgcn_perm(y[c], x[c], 0x05040100u);
+        o[2 * c + 1][p] = __builtin_amdgcn_perm(y[c], x[c], 0x07060302u);
       }
-      memcpy(&av, ta, 16);
-      memcpy(&bv, tb, 16);
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[t], 0, 0, 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+      *(uint4*)(tile + (8 * cb + c) * kWgStride + 8 * rb) = uint4{o[c][0], o[c][1], o[c][2], o[c][3]};
+    __syncthreads();
+    if (r0 + kWgRows < rend) load(r0 + kWgRows);
+#pragma unroll
+    for (int ks = 0; ks < kWgRows / 16; ks++) {
+      bf16x8 av[2], bv[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        av[i] = *(const bf16x8*)(tile + (m0 + 32 * i + col) * kWgStride + 16 * ks + 8 * half);
+        bv[i] = *(const bf16x8*)(tile + (128 + k0 + 32 * i + col) * kWgStride + 16 * ks + 8 * half);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+      if (bias) {
+        const bf16x8 one = __builtin_bit_cast(bf16x8, uint4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+#pragma unroll
+        for (int i = 0; i < 2; i++) accb[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], one, accb[i], 0, 0, 0);
+      }
     }
   }
-  float* out = a.partial + (int64_t)blockIdx.x * a.mg * K;
+  float* out = a.partial + (int64_t)blockIdx.x * 2 * 128 * 128 + hf.out;
 #pragma unroll
-  for (int t = 0; t < 8; t++) {
-    const int tile = w * 8 + t;
-    const int ti = tile / tk, tj = tile % tk;
+  for (int i = 0; i < 2; i++)
+#pragma unroll
     for (int v = 0; v < 16; v++) {
-      const int mrow = ti * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-      const int kcol = tj * 32 + (lane & 31);
-      out[(int64_t)mrow * K + kcol] = acc[t][v];
+      const int m = m0 + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
+#pragma unroll
+      for (int j = 0; j < 2; j++) out[(int64_t)m * a.ldo + k0 + 32 * j + col] = acc[i][j][v];
+      if (bias && col == 0) a.part_b[(int64_t)blockIdx.x * 128 + m] = accb[i][v];
     }
-  }
 }
 
-// out[k] = sum over p < np of partial[p][k], in order of p
-__global__ __launch_bounds__(256) void k_sum_partials(const float* __restrict__ partial, int np, int64_t len,
-                                                      float* __restrict__ out) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= len) return;
+// dst[k] = sum over p < np of src[p * len + k] in a fixed order, for every gradient of a backward pass in one launch:
+// each block takes 64 outputs of one segment, four threads per output each add a quarter of the partial sums (eight
+// loads in flight), then the four are added in order. One serial chain of np loads per output, a launch for each
+// gradient, took 97 us at np = 256 (17 launches per backward pass, 1.65 ms of 4.65 at 50k spheres); now one launch of
+// 28 us (104 MB of partial sums).
+struct RedSeg {
+  const float* src;
+  float* dst;
+  int np, len;
+  int block0;  // first block of the segment
+};
+constexpr int kMaxSeg = 24;
+struct RedArgs {
+  RedSeg seg[kMaxSeg];
+  int nseg;
+};
+__global__ __launch_bounds__(256) void k_reduce(RedArgs a) {
+  __shared__ float part[4][64];
+  int si = 0;
+  while (si + 1 < a.nseg && (int)blockIdx.x >= a.seg[si + 1].block0) si++;
+  const RedSeg sg = a.seg[si];
+  const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int64_t k = (int64_t)((int)blockIdx.x - sg.block0) * 64 + c;
+  const int per = (sg.np + 3) / 4, p0 = q * per, p1 = std::min(sg.np, p0 + per);
   float s = 0.f;
-  for (int p = 0; p < np; p++) s += partial[(int64_t)p * len + k];
-  out[k] = s;
-}
-
-// column sums of a bf16 [n][m] matrix (bias gradients): block b sums rows b, b+B, ... per column
-__global__ __launch_bounds__(256) void k_colsum(const uint16_t* __restrict__ gm, int64_t n, int m,
-                                                float* __restrict__ partial) {
-  for (int c = threadIdx.x; c < m; c += blockDim.x) {
-    float s = 0.f;
-    for (int64_t r = blockIdx.x; r < n; r += gridDim.x) s += bf2f(gm[r * m + c]);
-    partial[(int64_t)blockIdx.x * m + c] = s;
+  if (k < sg.len) {
+    const float* src = sg.src + k;
+    int p = p0;
+    for (; p + 8 <= p1; p += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = src[(int64_t)(p + u) * sg.len];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; p < p1; p++) s += src[(int64_t)p * sg.len];
   }
+  part[q][c] = s;
+  __syncthreads();
+  if (q == 0 && k < sg.len) sg.dst[k] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
 }
 
 // ------------------------------------------------------------------------------------- messages
@@ -479,7 +528,6 @@ struct MsgArgs {
   NbrList nl;
   const uint16_t* e;
   const uint16_t* pq;
-  const float* wE;  // [H][FE] rounded
   const float* bE;
   uint16_t* m;       // forward output [n][H]
   const float* dm;   // backward input [n][H]
@@ -621,8 +669,8 @@ __global__ __launch_bounds__(256) void k_msg_fwd_mfma(MsgArgs a, const uint16_t*
 //
 // The gates go to `gate` (128 bits per slot), so that the partner's side (k_msg_bwd_q) need not form z again.
 // Replaces one wavefront per particle with two channels per lane, which spent 250 vector instructions per edge
-// and one dependent chain of gathers per edge: 592 us per layer at 50k spheres (297k entries), now 45 us with
-// k_msg_bwd_q.
+// and one dependent chain of gathers per edge: 592 us per layer at 50k spheres (297k entries), now 65 us, and 28 us
+// for k_msg_bwd_q. Bound by the latency of the gathered Q rows at two wavefronts per SIMD (190 VGPRs).
 struct BwdStep {
   bool ok;
   uint4 e;
@@ -988,7 +1036,7 @@ __global__ __launch_bounds__(256) void k_relu_grad(int64_t len, const float* __r
 // encoder backward: dpre = dh * (h0 > 0); W_in and b_in gradients, per-block partials
 __global__ __launch_bounds__(256) void k_encode_bwd(int64_t n, const uint16_t* __restrict__ x,
                                                     const uint16_t* __restrict__ h0, const float* __restrict__ dh,
-                                                    float* __restrict__ part) {
+                                                    float* __restrict__ part_w, float* __restrict__ part_b) {
   __shared__ float red[4][H * (FN + 1)];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int c = 2 * lane;
@@ -1016,18 +1064,12 @@ __global__ __launch_bounds__(256) void k_encode_bwd(int64_t n, const uint16_t* _
     red[wv][(c + 1) * (FN + 1) + k] = g1[k];
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < H * (FN + 1); idx += blockDim.x)
-    part[(int64_t)blockIdx.x * H * (FN + 1) + idx] = ((red[0][idx] + red[1][idx]) + red[2][idx]) + red[3][idx];
-}
-
-// scatter a [blocks][H][FN+1] / [H][FE+1]-style interleaved reduction into weight and bias gradients
-__global__ __launch_bounds__(256) void k_split_wb(const float* __restrict__ sum, int rows, int cols,
-                                                  float* __restrict__ gw, float* __restrict__ gb) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= rows * (cols + 1)) return;
-  const int r = idx / (cols + 1), k = idx % (cols + 1);
-  if (k < cols) gw[r * cols + k] = sum[idx];
-  else gb[r] = sum[idx];
+  for (int idx = threadIdx.x; idx < H * (FN + 1); idx += blockDim.x) {
+    const float s = ((red[0][idx] + red[1][idx]) + red[2][idx]) + red[3][idx];
+    const int ch = idx / (FN + 1), k = idx % (FN + 1);
+    if (k < FN) part_w[(int64_t)blockIdx.x * H * FN + ch * FN + k] = s;
+    else part_b[(int64_t)blockIdx.x * H + ch] = s;
+  }
 }
 
 // Adam, then the bf16 working copy and its fp32 image
@@ -1184,7 +1226,7 @@ struct xdem_gnn {
   xdem_gnn_config cfg{};
   Off off{};
   float* p = nullptr;   // fp32 master parameters
-  float* g = nullptr;   // gradients
+  float* g = nullptr;   // gradients, then the loss
   float* m1 = nullptr;  // Adam moments
   float* m2 = nullptr;
   uint16_t* wbf = nullptr;   // bf16 copy (MFMA operands)
@@ -1207,9 +1249,8 @@ struct xdem_gnn {
   uint16_t* dpq = nullptr;
   uint32_t* mirror = nullptr;
   uint32_t* gate = nullptr;  // gates of the messages' backward pass (MsgArgs::gate)
-  float* partial = nullptr;  // partial sums of the reductions (sized once, never reallocated)
+  float* partial = nullptr;  // partial sums of a backward pass (training; sized once, never reallocated)
   int64_t cap_partial = 0;
-  float* dec_sum = nullptr;  // decoder reduction: dW_out, db_out, loss
   double* snap = nullptr;
   double* xs = nullptr;
   double* xf = nullptr;
@@ -1299,44 +1340,49 @@ int gemm_p(xdem_gnn* G, const GemmArgs& a) {
   return XDEM_OK;
 }
 
-int ensure_partial(xdem_gnn* G, int64_t floats) {
-  if (floats <= G->cap_partial) return XDEM_OK;
-  if (G->cap_partial > 0) return set_err(G->c, XDEM_ERR_CAPACITY, "gnn: partial-sum buffer too small");
-  int rc = galloc(G->c, &G->partial, floats);
-  if (rc) return rc;
-  G->cap_partial = floats;
-  return XDEM_OK;
-}
+// The gradients of one backward pass as segments of partial sums, added by one k_reduce at its end.
+struct Reduction {
+  xdem_gnn* G;
+  RedArgs a{};
+  int blocks = 0;
+  int64_t used = 0;  // floats of G->partial handed out
+  // room for np partial sums of len floats, to be added into dst; null when the buffer is exhausted
+  float* add(int np, int len, float* dst) {
+    if (used + (int64_t)np * len > G->cap_partial || a.nseg == kMaxSeg) return nullptr;
+    float* src = G->partial + used;
+    used += (int64_t)np * len;
+    a.seg[a.nseg++] = RedSeg{src, dst, np, len, blocks};
+    blocks += (len + 63) / 64;
+    return src;
+  }
+};
+int no_partial(xdem_gnn* G) { return set_err(G->c, XDEM_ERR_CAPACITY, "gnn: partial-sum buffer too small"); }
 
-// weight gradient of an mg x K matrix into grads[off]
-int wgrad(xdem_gnn* G, const uint16_t* gm, int mg, const uint16_t* x1, int k1, const uint16_t* x2, int k2,
-          int64_t goff) {
-  xdem_ctx* c = G->c;
-  const int64_t n = c->n;
-  const int K = k1 + k2;
-  int blocks = (int)std::min<int64_t>(256, std::max<int64_t>(1, (n + 63) / 64));
-  int64_t rpb = (n + blocks - 1) / blocks;
-  rpb = (rpb + 15) / 16 * 16;
-  blocks = (int)((n + rpb - 1) / rpb);
-  const int64_t len = (int64_t)mg * K;
-  int rc = ensure_partial(G, len * blocks);
-  if (rc) return rc;
-  WgradArgs a{n, gm, mg, x1, k1, x2, k2, rpb, G->partial};
-  hipLaunchKernelGGL(k_wgrad, dim3(blocks), dim3(256), 0, c->stream, a);
-  hipLaunchKernelGGL(k_sum_partials, dim3(nb(len, 256)), dim3(256), 0, c->stream, G->partial, blocks, len,
-                     G->g + goff);
-  XDEM_HIP(c, hipGetLastError());
+// Row chunks of the weight gradients: whole stages of 64 rows, at most kWgChunks chunks (two sets of blocks each, so
+// that 50k rows or more give every CU a block)
+int64_t wgrad_rows(int64_t n) {
+  const int64_t r = (n + kWgChunks - 1) / kWgChunks;
+  return (r + kWgRows - 1) / kWgRows * kWgRows;
+}
+// gradients of W_U [H][2H] = du^T [h | m] with its bias, and of W_AB [2H][H] = dpq^T h
+int wgrad_u(Reduction& R, const uint16_t* du, const uint16_t* h, const uint16_t* m, int64_t goff, int64_t boff) {
+  xdem_gnn* G = R.G;
+  const int64_t rpb = wgrad_rows(G->c->n);
+  const int blocks = nb(G->c->n, (int)rpb);
+  WgradArgs a{G->c->n, {{du, h, H, H, 0}, {du, m, H, H, H}}, H2, rpb, R.add(blocks, H * H2, G->g + goff),
+              R.add(blocks, H, G->g + boff)};
+  if (!a.partial || !a.part_b) return no_partial(G);
+  hipLaunchKernelGGL(k_wgrad, dim3(blocks, 2), dim3(256), 0, G->c->stream, a);
   return XDEM_OK;
 }
-int colsum(xdem_gnn* G, const uint16_t* gm, int m, int64_t goff) {
-  xdem_ctx* c = G->c;
-  const int blocks = (int)std::min<int64_t>(kRedBlocks, std::max<int64_t>(1, c->n));
-  int rc = ensure_partial(G, (int64_t)blocks * m);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(blocks), dim3(256), 0, c->stream, gm, c->n, m, G->partial);
-  hipLaunchKernelGGL(k_sum_partials, dim3(nb(m, 256)), dim3(256), 0, c->stream, G->partial, blocks, (int64_t)m,
-                     G->g + goff);
-  XDEM_HIP(c, hipGetLastError());
+int wgrad_ab(Reduction& R, const uint16_t* dpq, const uint16_t* h, int64_t goff) {
+  xdem_gnn* G = R.G;
+  const int64_t rpb = wgrad_rows(G->c->n);
+  const int blocks = nb(G->c->n, (int)rpb);
+  WgradArgs a{G->c->n, {{dpq, h, H2, H, 0}, {dpq + H, h, H2, H, (int64_t)H * H}}, H, rpb,
+              R.add(blocks, H * H2, G->g + goff), nullptr};
+  if (!a.partial) return no_partial(G);
+  hipLaunchKernelGGL(k_wgrad, dim3(blocks, 2), dim3(256), 0, G->c->stream, a);
   return XDEM_OK;
 }
 
@@ -1377,7 +1423,7 @@ int forward(xdem_gnn* G) {
     if ((rc = gemm_p<EPI_BF16, H2, H, 0>(G, g1))) return rc;
     MsgArgs ma{};
     ma.n = n; ma.nl = nl; ma.e = G->e; ma.pq = pq;
-    ma.wE = G->wr + G->off.W_E[l]; ma.bE = G->wr + G->off.b_E[l]; ma.m = mm;
+    ma.bE = G->wr + G->off.b_E[l]; ma.m = mm;
     hipLaunchKernelGGL(k_msg_fwd_mfma, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, c->stream, ma,
                        G->wbf + G->off.W_E[l]);
     GemmArgs g2{};
@@ -1412,23 +1458,18 @@ int backward(xdem_gnn* G, double* loss) {
   int rc;
   const NbrList& nl = c->nl[c->nl_cur];
   const int wgrid = (int)std::min<int64_t>(nb(n * 64, 256), kRedBlocks);
-  // decoder: loss, dh_L, dW_out, db_out
+  Reduction R{G};
+  // decoder: loss, dh_L, dW_out, db_out (contiguous, the loss right after the last parameter)
   const int dlen = FO * H + FO + 1;
-  if ((rc = ensure_partial(G, (int64_t)wgrid * dlen))) return rc;
-  DecArgs da{n, G->h[L], G->wr + G->off.W_out, G->wbf + G->off.W_out, G->wr + G->off.b_out, G->out, G->target, G->dh, G->partial};
+  float* dec = R.add(wgrid, dlen, G->g + G->off.W_out);
+  if (!dec) return no_partial(G);
+  DecArgs da{n, G->h[L], G->wr + G->off.W_out, G->wbf + G->off.W_out, G->wr + G->off.b_out, G->out, G->target, G->dh, dec};
   hipLaunchKernelGGL(k_decode<true>, dim3(wgrid), dim3(256), 0, c->stream, da);
-  // reduce into g[W_out..b_out] (contiguous) and the loss (one float after)
-  hipLaunchKernelGGL(k_sum_partials, dim3(nb(dlen, 256)), dim3(256), 0, c->stream, G->partial, wgrid, (int64_t)dlen,
-                     G->dec_sum);
-  XDEM_HIP(c, hipMemcpyAsync(G->g + G->off.W_out, G->dec_sum, sizeof(float) * (FO * H + FO), hipMemcpyDeviceToDevice,
-                             c->stream));
-  XDEM_HIP(c, hipMemcpyAsync(G->h_loss, G->dec_sum + FO * H + FO, sizeof(float), hipMemcpyDeviceToHost, c->stream));
   XDEM_HIP(c, hipGetLastError());
   for (int l = L - 1; l >= 0; l--) {
     // update: du, dW_U, db_U, dX -> dh (residual already in dh), dm
     hipLaunchKernelGGL(k_relu_grad, dim3(nb(n * H, 256)), dim3(256), 0, c->stream, n * H, G->dh, G->u[l], G->du);
-    if ((rc = wgrad(G, G->du, H, G->h[l], H, G->m[l], H, G->off.W_U[l]))) return rc;
-    if ((rc = colsum(G, G->du, H, G->off.b_U[l]))) return rc;
+    if ((rc = wgrad_u(R, G->du, G->h[l], G->m[l], G->off.W_U[l], G->off.b_U[l]))) return rc;
     uint16_t* tab = G->wT + (int64_t)l * 2 * H * H2;
     GemmArgs g1{};
     g1.n = n; g1.a1 = G->du; g1.k1 = H; g1.k2 = 0;
@@ -1437,21 +1478,18 @@ int backward(xdem_gnn* G, double* loss) {
     if ((rc = gemm_p<EPI_BWD_U, H2, H, 0>(G, g1))) return rc;
     // messages: dP|dQ, dW_E, db_E
     const int ngroups = nb(n, 32), mb = std::min(ngroups, kRedBlocks);
-    if ((rc = ensure_partial(G, (int64_t)mb * H * (FE + 1)))) return rc;
     MsgArgs ma{};
     ma.n = n; ma.nl = nl; ma.e = G->e; ma.pq = G->pq[l];
-    ma.wE = G->wr + G->off.W_E[l]; ma.bE = G->wr + G->off.b_E[l];
+    ma.bE = G->wr + G->off.b_E[l];
     ma.dm = G->dm; ma.mirror = G->mirror; ma.gate = G->gate; ma.dpq = G->dpq;
-    ma.part_w = G->partial; ma.part_b = G->partial + (int64_t)mb * H * FE;
+    ma.part_w = R.add(mb, H * FE, G->g + G->off.W_E[l]);
+    ma.part_b = R.add(mb, H, G->g + G->off.b_E[l]);
+    if (!ma.part_w || !ma.part_b) return no_partial(G);
     hipLaunchKernelGGL(k_msg_bwd, dim3(mb), dim3(256), 0, c->stream, ma, G->wbf + G->off.W_E[l], ngroups);
     hipLaunchKernelGGL(k_msg_bwd_q, dim3(nb(n, 4)), dim3(256), 0, c->stream, ma);
-    hipLaunchKernelGGL(k_sum_partials, dim3(nb((int64_t)H * FE, 256)), dim3(256), 0, c->stream, ma.part_w, mb,
-                       (int64_t)H * FE, G->g + G->off.W_E[l]);
-    hipLaunchKernelGGL(k_sum_partials, dim3(nb(H, 256)), dim3(256), 0, c->stream, ma.part_b, mb, (int64_t)H,
-                       G->g + G->off.b_E[l]);
     XDEM_HIP(c, hipGetLastError());
     // P|Q: dW_AB, dh += dPQ W_AB
-    if ((rc = wgrad(G, G->dpq, H2, G->h[l], H, nullptr, 0, G->off.W_AB[l]))) return rc;
+    if ((rc = wgrad_ab(R, G->dpq, G->h[l], G->off.W_AB[l]))) return rc;
     GemmArgs g2{};
     g2.n = n; g2.a1 = G->dpq; g2.k1 = H2; g2.k2 = 0;
     g2.b = tab;  // W_AB^T [H][2H]
@@ -1459,17 +1497,13 @@ int backward(xdem_gnn* G, double* loss) {
     if ((rc = gemm_p<EPI_ADD, H, H2, 0>(G, g2))) return rc;
   }
   // encoder
-  {
-    const int eb = wgrid;
-    const int64_t len = (int64_t)H * (FN + 1);
-    if ((rc = ensure_partial(G, eb * len + len))) return rc;
-    hipLaunchKernelGGL(k_encode_bwd, dim3(eb), dim3(256), 0, c->stream, n, G->x, G->h[0], G->dh, G->partial);
-    float* sum = G->partial + eb * len;
-    hipLaunchKernelGGL(k_sum_partials, dim3(nb(len, 256)), dim3(256), 0, c->stream, G->partial, eb, len, sum);
-    hipLaunchKernelGGL(k_split_wb, dim3(nb(len, 256)), dim3(256), 0, c->stream, sum, H, FN, G->g + G->off.W_in,
-                       G->g + G->off.b_in);
-    XDEM_HIP(c, hipGetLastError());
-  }
+  float* ew = R.add(wgrid, H * FN, G->g + G->off.W_in);
+  float* eb = R.add(wgrid, H, G->g + G->off.b_in);
+  if (!ew || !eb) return no_partial(G);
+  hipLaunchKernelGGL(k_encode_bwd, dim3(wgrid), dim3(256), 0, c->stream, n, G->x, G->h[0], G->dh, ew, eb);
+  hipLaunchKernelGGL(k_reduce, dim3(R.blocks), dim3(256), 0, c->stream, R.a);
+  XDEM_HIP(c, hipGetLastError());
+  XDEM_HIP(c, hipMemcpyAsync(G->h_loss, G->g + G->off.total, sizeof(float), hipMemcpyDeviceToHost, c->stream));
   XDEM_HIP(c, hipStreamSynchronize(c->stream));
   if (loss) *loss = (double)G->h_loss[0] / (double)(n * FO);
   return XDEM_OK;
@@ -1490,13 +1524,14 @@ extern "C" int xdem_gnn_create(xdem_ctx* c, const xdem_gnn_config* cfg, xdem_gnn
   G->off = offsets();
   const int64_t np = G->off.total;
   int rc;
-  if ((rc = galloc(c, &G->p, np)) || (rc = galloc(c, &G->g, np)) || (rc = galloc(c, &G->m1, np)) ||
+  if ((rc = galloc(c, &G->p, np)) || (rc = galloc(c, &G->g, np + 1)) || (rc = galloc(c, &G->m1, np)) ||
       (rc = galloc(c, &G->m2, np)) || (rc = galloc(c, &G->wbf, np)) || (rc = galloc(c, &G->wr, np)) ||
       (rc = galloc(c, &G->wT, (int64_t)L * 2 * H * H2)) || (rc = galloc(c, &G->dpart, 4 * 65536)) ||
-      (rc = galloc(c, &G->dec_sum, FO * H + FO + 1)) || (rc = ensure_partial(G, kPartialFloats))) {
+      (cfg->train && (rc = galloc(c, &G->partial, kPartialFloats)))) {
     delete G;
     return rc;
   }
+  G->cap_partial = cfg->train ? kPartialFloats : 0;
   XDEM_HIP(c, hipMemsetAsync(G->p, 0, sizeof(float) * np, c->stream));
   XDEM_HIP(c, hipMemsetAsync(G->g, 0, sizeof(float) * np, c->stream));
   XDEM_HIP(c, hipMemsetAsync(G->m1, 0, sizeof(float) * np, c->stream));
@@ -1516,7 +1551,7 @@ extern "C" int xdem_gnn_destroy(xdem_gnn* G) {
   (void)hipStreamSynchronize(G->c->stream);
   void* bufs[] = {G->p,  G->g,   G->m1,     G->m2,      G->wbf,     G->wr,      G->wT,
                   G->x,  G->e,   G->out,    G->target,  G->dh,      G->dm,      G->du,
-                  G->dpq, G->mirror, G->gate, G->partial, G->snap, G->xs, G->xf, G->dpart, G->dec_sum};
+                  G->dpq, G->mirror, G->gate, G->partial, G->snap, G->xs, G->xf, G->dpart};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (int k = 0; k <= L; k++)
