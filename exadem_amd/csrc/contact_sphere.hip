@@ -13,31 +13,9 @@
 #include <algorithm>
 #include <cmath>
 
-#include "contact_law.h"
-#include "mesh.h"
-#include "step.h"
+#include "contact_wide.h"
 
 namespace xdem {
-
-struct Q4f {
-  double w, x, y, z;
-};
-__device__ inline V3 qrot_d(Q4f q, V3 v) {
-  const V3 qv{q.x, q.y, q.z};
-  V3 uv = cross(qv, v);
-  V3 uuv = cross(qv, uv);
-  uv = uv * (2.0 * q.w);
-  uuv = uuv * 2.0;
-  return v + uv + uuv;
-}
-__device__ inline V3 angular_accel_d(Q4f Q, V3 mom, V3 vrot, V3 I) {
-  const Q4f Qi{Q.w, -Q.x, -Q.y, -Q.z};
-  const V3 om = qrot_d(Qi, vrot);
-  const V3 M = qrot_d(Qi, mom);
-  const V3 dom{(M.x - (I.z - I.y) * om.y * om.z) / I.x, (M.y - (I.x - I.z) * om.z * om.x) / I.y,
-               (M.z - (I.y - I.x) * om.x * om.y) / I.z};
-  return qrot_d(Q, dom);
-}
 
 struct ForceArgs {
   int64_t n;
@@ -100,6 +78,121 @@ __device__ inline void fetch_entry(const ForceArgs& a, uint64_t sl, uint32_t wd,
   }
 }
 
+// Entry e (list slot sl) of the particle `me`: detection, Hooke law and history; in contact, its force and moment are
+// added to F and M. An entry the partner owns is evaluated in the partner's orientation.
+template <bool KR, bool REC>
+__device__ __forceinline__ void pair_fp64(const ForceArgs& a, uint64_t sl, const Entry& e, const Own& me, V3& F, V3& M) {
+  const uint32_t wd = e.wd;
+  uint32_t* __restrict__ word = a.nl.word;
+  const V3 rx = me.r, vx = me.v, wx = me.w;
+  const double Rx = me.R, mx = me.m;
+  const bool owner = (wd & kOwnerBit) != 0;
+  V3 ri, rj;
+  double Ri, Rj;
+  if (owner) {
+    const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
+    ri = rx;
+    Ri = Rx;
+    rj = {e.p.x + sh.x, e.p.y + sh.y, e.p.z + sh.z};
+    Rj = e.p.w;
+  } else {
+    ri = {e.p.x, e.p.y, e.p.z};
+    Ri = e.p.w;
+    rj = rx;
+    Rj = Rx;
+  }
+  // detection_vertex_vertex_core
+  const V3 dist = ri - rj;
+  const double dnorm = norm(dist);
+  const double dn = dnorm - (Ri + Rj);
+  if (dn < 0) {
+    const double inv = 1.0 / dnorm;
+    const V3 nrm = dist * inv;
+    const V3 cpos = ri - nrm * (Ri + 0.5 * dn);
+    const V3 vy{e.v.x, e.v.y, e.v.z}, wy{e.w.x, e.w.y, e.w.z};
+    const double my = e.v.w;
+    const double mi = owner ? mx : my, mj = owner ? my : mx;
+    const double meff = (mi * mj) / (mi + mj);
+    V3 ft = e.ft;
+    V3 mint = e.mint;
+    const V3 f = owner ? hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vx, wx, rj, vy, wy)
+                       : hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vy, wy, rj, vx, wx);
+    if (REC && a.cstate && owner) {
+      // the tuple the reference's functor returns for analyses: dn, contact point, f - ft, ft
+      // (contact_sphere.hpp:175-202), with the two positions the interaction dump writes
+      const V3 fnv = f - ft;
+      const double rec[kCStateLen] = {dn,   cpos.x, cpos.y, cpos.z, fnv.x, fnv.y, fnv.z, ft.x,
+                                      ft.y, ft.z,   ri.x,   ri.y,   ri.z,   rj.x,  rj.y,  rj.z};
+      double* r = a.cstate + (uint64_t)kCStateLen * sl;
+#pragma unroll
+      for (int q = 0; q < kCStateLen; q++) r[q] = rec[q];
+    }
+    const bool act = !(ft.x == 0 && ft.y == 0 && ft.z == 0 && mint.x == 0 && mint.y == 0 && mint.z == 0);
+    if (act || (wd & kActiveBit)) {
+      a.nl.hx[sl] = ft.x;
+      a.nl.hy[sl] = ft.y;
+      a.nl.hz[sl] = ft.z;
+      if (KR) {
+        a.nl.mhx[sl] = mint.x;
+        a.nl.mhy[sl] = mint.y;
+        a.nl.mhz[sl] = mint.z;
+      }
+    }
+    const uint32_t nwd = act ? (wd | kActiveBit) : (wd & ~kActiveBit);
+    if (nwd != wd) word[sl] = nwd;
+    if (owner) {
+      F = F + f;
+      M = M + (cross(cpos - rx, f) + mint);
+    } else {
+      const V3 nf = -f;
+      M = M + (cross(cpos - rx, nf) + (-mint));
+      F = F + nf;
+    }
+  } else {
+    if (wd & kActiveBit) {
+      a.nl.hx[sl] = 0.0;
+      a.nl.hy[sl] = 0.0;
+      a.nl.hz[sl] = 0.0;
+      if (KR) {
+        a.nl.mhx[sl] = 0.0;
+        a.nl.mhy[sl] = 0.0;
+        a.nl.mhz[sl] = 0.0;
+      }
+      word[sl] = wd & ~kActiveBit;
+    }
+    if (REC && a.cstate && owner) {
+      // no contact: dn reported 0, no forces (contact_sphere.hpp:197-200); the dump skips the entry
+      double* r = a.cstate + (uint64_t)kCStateLen * sl;
+#pragma unroll
+      for (int q = 0; q < kCStateLen; q++) r[q] = 0.0;
+    }
+  }
+}
+
+// The several-lanes pass (contact_wide.h) with this form's pairs
+template <bool KR>
+struct WideFp64 {
+  typedef ForceArgs Args;
+  typedef xdem::Entry Entry;
+  typedef double T;
+  static constexpr bool kKr = KR;
+  struct Acc {
+    double v;
+    __device__ void init(double x) { v = x; }
+    __device__ void add(double x) { v = v + x; }
+    __device__ double value() const { return v; }
+  };
+  static __device__ inline void fetch(const Args& a, uint64_t sl, uint32_t wd, Entry& e) {
+    fetch_entry<KR>(a, sl, wd, e, nullptr, kNoTile);
+  }
+  static __device__ inline void eval(const Args& a, uint64_t sl, const Entry& e, const Own& me, double (&c)[6]) {
+    V3 f{c[0], c[1], c[2]}, m{c[3], c[4], c[5]};  // -0.0, to which any value adds as itself
+    pair_fp64<KR, false>(a, sl, e, me, f, m);
+    c[0] = f.x; c[1] = f.y; c[2] = f.z;
+    c[3] = m.x; c[4] = m.y; c[5] = m.z;
+  }
+};
+
 // INTEG (with FUSED): after the particle's force, its epilog kick and the prolog of the next step
 // are applied and the next record is written to core_out, with the displacement test of the rebuild
 // trigger; accelerations, moments and angular accelerations are then not stored (the next pass
@@ -139,11 +232,11 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
   uint32_t wd2 = 0;
   if (cnt > 0) fetch_entry<KR>(a, b, word[b], nxt, tile, b0);
   if (cnt > 1) wd2 = word[b + kWave];
-  const Core me = tile[threadIdx.x];
-  const V3 rx{me.xr.x, me.xr.y, me.xr.z};
-  const V3 vx{me.vm.x, me.vm.y, me.vm.z};
-  const V3 wx{me.w.x, me.w.y, me.w.z};
-  const double mx = me.vm.w, Rx = me.xr.w;
+  const Core rec = tile[threadIdx.x];
+  const Own me{V3{rec.xr.x, rec.xr.y, rec.xr.z}, rec.xr.w, V3{rec.vm.x, rec.vm.y, rec.vm.z},
+               V3{rec.w.x, rec.w.y, rec.w.z}, rec.vm.w};
+  const V3 rx = me.r, vx = me.v, wx = me.w;
+  const double mx = me.m, Rx = me.R;
   V3 F, M;
   if (FUSED) {
     F = {0.0, 0.0, 0.0};
@@ -160,89 +253,8 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
       fetch_entry<KR>(a, sl + kWave, wd2, nxt, tile, b0);
       if (k + 2 < cnt) wd2 = word[sl + 2 * kWave];
     }
-    const uint32_t wd = e.wd;
-    partner_tile(tile, b0, wd & kIdxMask, e.p, e.v, e.w);
-    const bool owner = (wd & kOwnerBit) != 0;
-    V3 ri, rj;
-    double Ri, Rj;
-    if (owner) {
-      const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
-      ri = rx;
-      Ri = Rx;
-      rj = {e.p.x + sh.x, e.p.y + sh.y, e.p.z + sh.z};
-      Rj = e.p.w;
-    } else {
-      ri = {e.p.x, e.p.y, e.p.z};
-      Ri = e.p.w;
-      rj = rx;
-      Rj = Rx;
-    }
-    // detection_vertex_vertex_core
-    const V3 dist = ri - rj;
-    const double dnorm = norm(dist);
-    const double dn = dnorm - (Ri + Rj);
-    if (dn < 0) {
-      const double inv = 1.0 / dnorm;
-      const V3 nrm = dist * inv;
-      const V3 cpos = ri - nrm * (Ri + 0.5 * dn);
-      const V3 vy{e.v.x, e.v.y, e.v.z}, wy{e.w.x, e.w.y, e.w.z};
-      const double my = e.v.w;
-      const double mi = owner ? mx : my, mj = owner ? my : mx;
-      const double meff = (mi * mj) / (mi + mj);
-      V3 ft = e.ft;
-      V3 mint = e.mint;
-      const V3 f = owner ? hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vx, wx, rj, vy, wy)
-                         : hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vy, wy, rj, vx, wx);
-      if (!INTEG && a.cstate && owner) {
-        // the tuple the reference's functor returns for analyses: dn, contact point, f - ft, ft
-        // (contact_sphere.hpp:175-202), with the two positions the interaction dump writes
-        const V3 fnv = f - ft;
-        const double rec[kCStateLen] = {dn,   cpos.x, cpos.y, cpos.z, fnv.x, fnv.y, fnv.z, ft.x,
-                                        ft.y, ft.z,   ri.x,   ri.y,   ri.z,   rj.x,  rj.y,  rj.z};
-        double* r = a.cstate + (uint64_t)kCStateLen * sl;
-#pragma unroll
-        for (int q = 0; q < kCStateLen; q++) r[q] = rec[q];
-      }
-      const bool act = !(ft.x == 0 && ft.y == 0 && ft.z == 0 && mint.x == 0 && mint.y == 0 && mint.z == 0);
-      if (act || (wd & kActiveBit)) {
-        a.nl.hx[sl] = ft.x;
-        a.nl.hy[sl] = ft.y;
-        a.nl.hz[sl] = ft.z;
-        if (KR) {
-          a.nl.mhx[sl] = mint.x;
-          a.nl.mhy[sl] = mint.y;
-          a.nl.mhz[sl] = mint.z;
-        }
-      }
-      const uint32_t nwd = act ? (wd | kActiveBit) : (wd & ~kActiveBit);
-      if (nwd != wd) word[sl] = nwd;
-      if (owner) {
-        F = F + f;
-        M = M + (cross(cpos - rx, f) + mint);
-      } else {
-        const V3 nf = -f;
-        M = M + (cross(cpos - rx, nf) + (-mint));
-        F = F + nf;
-      }
-    } else {
-      if (wd & kActiveBit) {
-        a.nl.hx[sl] = 0.0;
-        a.nl.hy[sl] = 0.0;
-        a.nl.hz[sl] = 0.0;
-        if (KR) {
-          a.nl.mhx[sl] = 0.0;
-          a.nl.mhy[sl] = 0.0;
-          a.nl.mhz[sl] = 0.0;
-        }
-        word[sl] = wd & ~kActiveBit;
-      }
-      if (!INTEG && a.cstate && owner) {
-        // no contact: dn reported 0, no forces (contact_sphere.hpp:197-200); the dump skips the entry
-        double* r = a.cstate + (uint64_t)kCStateLen * sl;
-#pragma unroll
-        for (int q = 0; q < kCStateLen; q++) r[q] = 0.0;
-      }
-    }
+    partner_tile(tile, b0, e.wd & kIdxMask, e.p, e.v, e.w);
+    pair_fp64<KR, !INTEG>(a, sl, e, me, F, M);
   }
   // the integration's own inputs (inertia, rebuild reference), loaded before the walls and the mesh terms
   // so that their latency overlaps with those
@@ -293,8 +305,8 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
   }
   if (MESH && mwave) mesh_add_at(a.mt, midx, F, M);
   if (FUSED && INTEG) {
-    const V3 al = angular_accel_d(Q4f{me.q.x, me.q.y, me.q.z, me.q.w}, M, wx, inert);
-    Core nx = me;
+    const V3 al = angular_accel(Q4{rec.q.x, rec.q.y, rec.q.z, rec.q.w}, M, wx, inert);
+    Core nx = rec;
     kick_prolog<true>(nx.xr, nx.vm, nx.w, nx.q, F.x / mx, F.y / mx, F.z / mx, al.x, al.y, al.z, a.dt, a.kdt_2);
     a.core_out[x] = nx;
     const double dx = nx.xr.x - bref.x, dy = nx.xr.y - bref.y, dz = nx.xr.z - bref.z;
@@ -307,7 +319,7 @@ __global__ __launch_bounds__(256) void k_force_fp64(ForceArgs a) {
     s.my[x] = M.y;
     s.mz[x] = M.z;
     const d4 q = s.core[x].q;
-    const V3 al = angular_accel_d(Q4f{q.x, q.y, q.z, q.w}, M, wx, V3{s.ix[x], s.iy[x], s.iz[x]});
+    const V3 al = angular_accel(Q4{q.x, q.y, q.z, q.w}, M, wx, V3{s.ix[x], s.iy[x], s.iz[x]});
     s.alx[x] = al.x;
     s.aly[x] = al.y;
     s.alz[x] = al.z;
@@ -349,6 +361,16 @@ int launch_force_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams&
 int launch_step_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, bool gravity_on, V3 g,
                      double thr2, int32_t step_tag, Core** input);
 
+// After an integrating pass: its output becomes the live records.
+int finish_step(xdem_ctx* c, int32_t trig_out, Core** input) {
+  XDEM_HIP(c, hipGetLastError());
+  c->cs_valid = false;  // the integrating pass does not record
+  *input = live(c).core;
+  std::swap(live(c).core, c->core_alt);
+  c->trig_slot = trig_out;
+  return XDEM_OK;
+}
+
 int launch_step(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, int form, bool gravity_on,
                 V3 g, double thr2, int32_t step_tag, Core** input) {
   *input = nullptr;
@@ -382,6 +404,11 @@ int launch_step(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, 
   a.core_out = c->core_alt;
   a.kdt_2 = dt * 0.5;
   a.thr2 = thr2;
+  if (const int lanes = wide_lanes(a.n, c->nl_max_rows); lanes > 1) {
+    if (c->kr_used) launch_wide<WideFp64<true>>(c, a, lanes, true, true, true);
+    else launch_wide<WideFp64<false>>(c, a, lanes, true, true, true);
+    return finish_step(c, a.trig_out, input);
+  }
   const dim3 grid(grid_blocks(a.n, 256)), block(256);
   // engine step: drivers and mesh terms each only when present
 #define STEP(KRV, W, M) hipLaunchKernelGGL((k_force_fp64<true, KRV, W, true, true, M>), grid, block, 0, c->stream, a)
@@ -393,12 +420,7 @@ int launch_step(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, 
     else { if (meshed) STEP(false, false, true); else STEP(false, false, false); }
   }
 #undef STEP
-  XDEM_HIP(c, hipGetLastError());
-  c->cs_valid = false;  // the integrating pass does not record
-  *input = live(c).core;
-  std::swap(live(c).core, c->core_alt);
-  c->trig_slot = a.trig_out;
-  return XDEM_OK;
+  return finish_step(c, a.trig_out, input);
 }
 
 int launch_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, int form, bool fused,
@@ -456,7 +478,11 @@ int launch_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd,
     }
   }
   if (meshed && (rc = launch_mesh_pass(c, cpd, dt, guarded, c->trig_slot, mstate, &a.mt))) return rc;
-  if (fused) launch_f<true>(c, a, c->kr_used, walls, guarded);
+  const int lanes = wide_lanes(a.n, c->nl_max_rows);
+  if (lanes > 1 && !c->record_cs && (fused || !guarded)) {
+    if (c->kr_used) launch_wide<WideFp64<true>>(c, a, lanes, fused, false, guarded);
+    else launch_wide<WideFp64<false>>(c, a, lanes, fused, false, guarded);
+  } else if (fused) launch_f<true>(c, a, c->kr_used, walls, guarded);
   else launch_f<false>(c, a, c->kr_used, walls, guarded);
   XDEM_HIP(c, hipGetLastError());
   c->cs_valid = c->record_cs;

@@ -8,9 +8,7 @@
 // src/forcefield/include/exaDEM/forcefield/contact_force.hpp:146-235) and the friction history (12 bytes
 // per slot instead of 24). Per-particle sums of the contact forces and moments are accumulated in FP32
 // with TwoSum compensation and added to the FP64 gravity term at the end.
-#include "contact_law.h"
-#include "mesh.h"
-#include "step.h"
+#include "contact_wide.h"
 
 namespace xdem {
 
@@ -103,26 +101,6 @@ struct ForceArgs32 {
 };
 
 
-struct Q4g {
-  double w, x, y, z;
-};
-__device__ inline V3 qrot_g(Q4g q, V3 v) {
-  const V3 qv{q.x, q.y, q.z};
-  V3 uv = cross(qv, v);
-  V3 uuv = cross(qv, uv);
-  uv = uv * (2.0 * q.w);
-  uuv = uuv * 2.0;
-  return v + uv + uuv;
-}
-__device__ inline V3 angular_accel_g(Q4g Q, V3 mom, V3 vrot, V3 I) {
-  const Q4g Qi{Q.w, -Q.x, -Q.y, -Q.z};
-  const V3 om = qrot_g(Qi, vrot);
-  const V3 M = qrot_g(Qi, mom);
-  const V3 dom{(M.x - (I.z - I.y) * om.y * om.z) / I.x, (M.y - (I.x - I.z) * om.z * om.x) / I.y,
-               (M.z - (I.y - I.x) * om.x * om.y) / I.z};
-  return qrot_g(Q, dom);
-}
-
 struct Entry32 {
   uint32_t wd;
   d4 p;
@@ -148,6 +126,118 @@ __device__ inline void fetch32(const ForceArgs32& a, uint64_t sl, uint32_t wd, E
     e.mint = {0.0f, 0.0f, 0.0f};
   }
 }
+
+// Entry e (list slot sl) of the particle `me`: the FP64 sign test, FP32 geometry, law and history; in contact, the force
+// and moment the particle adds go to add(force, moment). An entry the partner owns is evaluated in the partner's
+// orientation. vx, wx, mxf: the particle's velocity, spin and mass rounded to FP32.
+template <bool KR, class Add>
+__device__ __forceinline__ void pair_fp32(const ForceArgs32& a, uint64_t sl, const Entry32& e, V3 rx, double Rx, F3 vx,
+                                          F3 wx, float mxf, Add&& add) {
+  uint32_t* __restrict__ word = a.nl.word;
+  const uint32_t wd = e.wd;
+  const bool owner = (wd & kOwnerBit) != 0;
+  V3 ri, rj;
+  double Ri, Rj;
+  if (owner) {
+    const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
+    ri = rx;
+    Ri = Rx;
+    rj = {e.p.x + sh.x, e.p.y + sh.y, e.p.z + sh.z};
+    Rj = e.p.w;
+  } else {
+    ri = {e.p.x, e.p.y, e.p.z};
+    Ri = e.p.w;
+    rj = rx;
+    Rj = Rx;
+  }
+  // FP64 overlap sign test: the contact set is the plain form's
+  const V3 dist = ri - rj;
+  const double dnorm = sqrt(dot(dist, dist));
+  const double dn = dnorm - (Ri + Rj);
+  if (dn < 0) {
+    const F3 d = to_f3(dist.x, dist.y, dist.z);
+    const float dnf = (float)dn;
+    const float inv = 1.0f / (float)dnorm;
+    const F3 nrm = d * inv;
+    const F3 bi = -(nrm * ((float)Ri + 0.5f * dnf));  // cp - ri
+    const F3 bj = bi + d;                            // cp - rj
+    const F3 vy = to_f3(e.v.x, e.v.y, e.v.z);
+    const F3 wy = to_f3(e.w.x, e.w.y, e.w.z);
+    const float my = (float)e.v.w;
+    const float mi = owner ? mxf : my, mj = owner ? my : mxf;
+    const float meff = (mi * mj) / (mi + mj);
+    F3 ft = e.ft;
+    F3 mint = e.mint;
+    const F3 f = owner ? hooke_force_f32<KR>(dnf, nrm, a.dtf, a.cp, meff, ft, mint, bi, bj, vx, wx, vy, wy)
+                       : hooke_force_f32<KR>(dnf, nrm, a.dtf, a.cp, meff, ft, mint, bi, bj, vy, wy, vx, wx);
+    const bool act = !(ft.x == 0 && ft.y == 0 && ft.z == 0 && mint.x == 0 && mint.y == 0 && mint.z == 0);
+    if (act || (wd & kActiveBit)) {
+      a.nl.fx32[sl] = ft.x;
+      a.nl.fy32[sl] = ft.y;
+      a.nl.fz32[sl] = ft.z;
+      if (KR) {
+        a.nl.mfx32[sl] = mint.x;
+        a.nl.mfy32[sl] = mint.y;
+        a.nl.mfz32[sl] = mint.z;
+      }
+    }
+    const uint32_t nwd = act ? (wd | kActiveBit) : (wd & ~kActiveBit);
+    if (nwd != wd) word[sl] = nwd;
+    // Both contact arms are parallel to n, so the normal force has no moment about either centre:
+    // (cp - r) x f = (cp - r) x ft exactly. The FP64 form evaluates the full product, whose normal
+    // part there is round-off of ~1e-16 |b| |fn|; in FP32 the same round-off (~1e-7 |b| |fn|) would
+    // swamp the friction moment, so only the tangential part enters.
+    F3 fc, tc;
+    if (owner) {
+      fc = f;
+      tc = crossf(bi, ft) + mint;
+    } else {
+      fc = -f;
+      tc = crossf(bj, -ft) + (-mint);
+    }
+    add(fc, tc);
+  } else if (wd & kActiveBit) {
+    a.nl.fx32[sl] = 0.0f;
+    a.nl.fy32[sl] = 0.0f;
+    a.nl.fz32[sl] = 0.0f;
+    if (KR) {
+      a.nl.mfx32[sl] = 0.0f;
+      a.nl.mfy32[sl] = 0.0f;
+      a.nl.mfz32[sl] = 0.0f;
+    }
+    word[sl] = wd & ~kActiveBit;
+  }
+}
+
+// The several-lanes pass (contact_wide.h) with this form's pairs: the FP32 terms are added with TwoSum compensation in
+// list order, then to the FP64 start value
+template <bool KR>
+struct WideFp32 {
+  typedef ForceArgs32 Args;
+  typedef Entry32 Entry;
+  typedef float T;
+  static constexpr bool kKr = KR;
+  struct Acc {
+    double base;
+    CSum s;
+    __device__ void init(double x) {
+      base = x;
+      s = CSum{0.0f, 0.0f};
+    }
+    __device__ void add(float x) { cadd(s, x); }
+    __device__ double value() const { return base + cval(s); }
+  };
+  static __device__ inline void fetch(const Args& a, uint64_t sl, uint32_t wd, Entry& e) {
+    fetch32<KR>(a, sl, wd, e, nullptr, kNoTile);
+  }
+  static __device__ inline void eval(const Args& a, uint64_t sl, const Entry& e, const Own& me, float (&c)[6]) {
+    pair_fp32<KR>(a, sl, e, me.r, me.R, to_f3(me.v.x, me.v.y, me.v.z), to_f3(me.w.x, me.w.y, me.w.z), (float)me.m,
+                  [&](F3 f, F3 m) {
+                    c[0] = f.x; c[1] = f.y; c[2] = f.z;
+                    c[3] = m.x; c[4] = m.y; c[5] = m.z;
+                  });
+  }
+};
 
 // INTEG (with FUSED): as k_force_fp64's integrating pass, the kick and next prolog of each particle
 // go to core_out right after its force.
@@ -201,85 +291,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       fetch32<KR>(a, sl + kWave, wd2, nxt, tile, b0);
       if (k + 2 < cnt) wd2 = word[sl + 2 * kWave];
     }
-    const uint32_t wd = e.wd;
-    partner_tile(tile, b0, wd & kIdxMask, e.p, e.v, e.w);
-    const bool owner = (wd & kOwnerBit) != 0;
-    V3 ri, rj;
-    double Ri, Rj;
-    if (owner) {
-      const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
-      ri = rx;
-      Ri = Rx;
-      rj = {e.p.x + sh.x, e.p.y + sh.y, e.p.z + sh.z};
-      Rj = e.p.w;
-    } else {
-      ri = {e.p.x, e.p.y, e.p.z};
-      Ri = e.p.w;
-      rj = rx;
-      Rj = Rx;
-    }
-    // FP64 overlap sign test: the contact set is the plain form's
-    const V3 dist = ri - rj;
-    const double dnorm = sqrt(dot(dist, dist));
-    const double dn = dnorm - (Ri + Rj);
-    if (dn < 0) {
-      const F3 d = to_f3(dist.x, dist.y, dist.z);
-      const float dnf = (float)dn;
-      const float inv = 1.0f / (float)dnorm;
-      const F3 nrm = d * inv;
-      const F3 bi = -(nrm * ((float)Ri + 0.5f * dnf));  // cp - ri
-      const F3 bj = bi + d;                            // cp - rj
-      const F3 vy = to_f3(e.v.x, e.v.y, e.v.z);
-      const F3 wy = to_f3(e.w.x, e.w.y, e.w.z);
-      const float my = (float)e.v.w;
-      const float mi = owner ? mxf : my, mj = owner ? my : mxf;
-      const float meff = (mi * mj) / (mi + mj);
-      F3 ft = e.ft;
-      F3 mint = e.mint;
-      const F3 f = owner ? hooke_force_f32<KR>(dnf, nrm, a.dtf, a.cp, meff, ft, mint, bi, bj, vx, wx, vy, wy)
-                         : hooke_force_f32<KR>(dnf, nrm, a.dtf, a.cp, meff, ft, mint, bi, bj, vy, wy, vx, wx);
-      const bool act = !(ft.x == 0 && ft.y == 0 && ft.z == 0 && mint.x == 0 && mint.y == 0 && mint.z == 0);
-      if (act || (wd & kActiveBit)) {
-        a.nl.fx32[sl] = ft.x;
-        a.nl.fy32[sl] = ft.y;
-        a.nl.fz32[sl] = ft.z;
-        if (KR) {
-          a.nl.mfx32[sl] = mint.x;
-          a.nl.mfy32[sl] = mint.y;
-          a.nl.mfz32[sl] = mint.z;
-        }
-      }
-      const uint32_t nwd = act ? (wd | kActiveBit) : (wd & ~kActiveBit);
-      if (nwd != wd) word[sl] = nwd;
-      // Both contact arms are parallel to n, so the normal force has no moment about either centre:
-      // (cp - r) x f = (cp - r) x ft exactly. The FP64 form evaluates the full product, whose normal
-      // part there is round-off of ~1e-16 |b| |fn|; in FP32 the same round-off (~1e-7 |b| |fn|) would
-      // swamp the friction moment, so only the tangential part enters.
-      F3 fc, tc;
-      if (owner) {
-        fc = f;
-        tc = crossf(bi, ft) + mint;
-      } else {
-        fc = -f;
-        tc = crossf(bj, -ft) + (-mint);
-      }
+    partner_tile(tile, b0, e.wd & kIdxMask, e.p, e.v, e.w);
+    pair_fp32<KR>(a, sl, e, rx, Rx, vx, wx, mxf, [&](F3 fc, F3 tc) {
       cadd(Fx, fc.x);
       cadd(Fy, fc.y);
       cadd(Fz, fc.z);
       cadd(Mx, tc.x);
       cadd(My, tc.y);
       cadd(Mz, tc.z);
-    } else if (wd & kActiveBit) {
-      a.nl.fx32[sl] = 0.0f;
-      a.nl.fy32[sl] = 0.0f;
-      a.nl.fz32[sl] = 0.0f;
-      if (KR) {
-        a.nl.mfx32[sl] = 0.0f;
-        a.nl.mfy32[sl] = 0.0f;
-        a.nl.mfz32[sl] = 0.0f;
-      }
-      word[sl] = wd & ~kActiveBit;
-    }
+    });
   }
   V3 F, M;
   if (FUSED) {
@@ -328,7 +348,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   }
   if (MESH && mwave) mesh_add_at(a.mt, midx, F, M);
   if (FUSED && INTEG) {
-    const V3 al = angular_accel_g(Q4g{me.q.x, me.q.y, me.q.z, me.q.w}, M, V3{me.w.x, me.w.y, me.w.z}, inert);
+    const V3 al = angular_accel(Q4{me.q.x, me.q.y, me.q.z, me.q.w}, M, V3{me.w.x, me.w.y, me.w.z}, inert);
     Core nx = me;
     kick_prolog<true>(nx.xr, nx.vm, nx.w, nx.q, F.x / mx, F.y / mx, F.z / mx, al.x, al.y, al.z, a.dt, a.kdt_2);
     a.core_out[x] = nx;
@@ -343,7 +363,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     s.mz[x] = M.z;
     const d4 q = me.q;
     const V3 al =
-        angular_accel_g(Q4g{q.x, q.y, q.z, q.w}, M, V3{me.w.x, me.w.y, me.w.z}, V3{s.ix[x], s.iy[x], s.iz[x]});
+        angular_accel(Q4{q.x, q.y, q.z, q.w}, M, V3{me.w.x, me.w.y, me.w.z}, V3{s.ix[x], s.iy[x], s.iz[x]});
     s.alx[x] = al.x;
     s.aly[x] = al.y;
     s.alz[x] = al.z;
@@ -427,7 +447,11 @@ int launch_force_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams&
   a.step_tag = step_tag;
   a.trig_in = c->trig_slot;
   const bool kr = c->kr_used;
-  if (fused) {
+  const int lanes = wide_lanes(a.n, c->nl_max_rows);
+  if (lanes > 1 && (fused || !guarded)) {
+    if (kr) launch_wide<WideFp32<true>>(c, a, lanes, fused, false, guarded);
+    else launch_wide<WideFp32<false>>(c, a, lanes, fused, false, guarded);
+  } else if (fused) {
     if (kr) walls ? launch32<true, true, true>(c, a, guarded) : launch32<true, true, false>(c, a, guarded);
     else walls ? launch32<true, false, true>(c, a, guarded) : launch32<true, false, false>(c, a, guarded);
   } else {
@@ -471,6 +495,11 @@ int launch_step_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams& 
   a.core_out = c->core_alt;
   a.kdt_2 = dt * 0.5;
   a.thr2 = thr2;
+  if (const int lanes = wide_lanes(a.n, c->nl_max_rows); lanes > 1) {
+    if (c->kr_used) launch_wide<WideFp32<true>>(c, a, lanes, true, true, true);
+    else launch_wide<WideFp32<false>>(c, a, lanes, true, true, true);
+    return finish_step(c, a.trig_out, input);
+  }
   const dim3 grid(grid_blocks(a.n, 256)), block(256);
 #define STEP(KRV, W, M) hipLaunchKernelGGL((k_force_fp32<true, KRV, W, true, true, M>), grid, block, 0, c->stream, a)
   if (c->kr_used) {
@@ -481,12 +510,7 @@ int launch_step_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams& 
     else { if (meshed) STEP(false, false, true); else STEP(false, false, false); }
   }
 #undef STEP
-  XDEM_HIP(c, hipGetLastError());
-  *input = live(c).core;
-  std::swap(live(c).core, c->core_alt);
-  c->trig_slot = a.trig_out;
-  c->cs_valid = false;  // the FP32 form does not record
-  return XDEM_OK;
+  return finish_step(c, a.trig_out, input);
 }
 
 }  // namespace xdem

@@ -11,26 +11,6 @@
 
 namespace xdem {
 
-// quat * vec3 (src/shape/include/exaDEM/type/quat.hpp:84-91)
-__device__ inline V3 qrot(Q4 q, V3 v) {
-  const V3 qv{q.x, q.y, q.z};
-  V3 uv = cross(qv, v);
-  V3 uuv = cross(qv, uv);
-  uv = uv * (2.0 * q.w);
-  uuv = uuv * 2.0;
-  return v + uv + uuv;
-}
-
-// PushToAngularAccelerationFunctor (src/numericalscheme/include/exaDEM/angular_acceleration.hpp:28-42)
-__device__ inline V3 angular_accel(Q4 Q, V3 mom, V3 vrot, V3 I) {
-  const Q4 Qi{Q.w, -Q.x, -Q.y, -Q.z};
-  const V3 om = qrot(Qi, vrot);
-  const V3 M = qrot(Qi, mom);
-  const V3 dom{(M.x - (I.z - I.y) * om.y * om.z) / I.x, (M.y - (I.x - I.z) * om.z * om.x) / I.y,
-               (M.z - (I.y - I.x) * om.x * om.y) / I.z};
-  return qrot(Q, dom);
-}
-
 // The 128-byte records of a block's 256 particles are moved between HBM and LDS with fully
 // coalesced 16-byte accesses (a record-per-lane access pattern would touch 64 lines per
 // instruction). LDS rows are padded to 144 bytes to spread the per-lane reads over the banks.

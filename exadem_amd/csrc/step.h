@@ -26,6 +26,26 @@ __device__ inline Q4 qnormalize(Q4 q) {
   return {q.w / n, q.x / n, q.y / n, q.z / n};
 }
 
+// quat * vec3 (src/shape/include/exaDEM/type/quat.hpp:84-91)
+__device__ inline V3 qrot(Q4 q, V3 v) {
+  const V3 qv{q.x, q.y, q.z};
+  V3 uv = cross(qv, v);
+  V3 uuv = cross(qv, uv);
+  uv = uv * (2.0 * q.w);
+  uuv = uuv * 2.0;
+  return v + uv + uuv;
+}
+
+// PushToAngularAccelerationFunctor (src/numericalscheme/include/exaDEM/angular_acceleration.hpp:28-42)
+__device__ inline V3 angular_accel(Q4 Q, V3 mom, V3 vrot, V3 I) {
+  const Q4 Qi{Q.w, -Q.x, -Q.y, -Q.z};
+  const V3 om = qrot(Qi, vrot);
+  const V3 M = qrot(Qi, mom);
+  const V3 dom{(M.x - (I.z - I.y) * om.y * om.z) / I.x, (M.y - (I.x - I.z) * om.z * om.x) / I.y,
+               (M.z - (I.y - I.x) * om.x * om.y) / I.z};
+  return qrot(Q, dom);
+}
+
 // Kick of the finished step (KICK) then the prolog of the next one, on one particle's record
 // (xr = position + radius, vm = velocity + mass, w = angular velocity + homothety, qq = orientation
 // stored {w, x, y, z} in {x, y, z, w}); a and al are the acceleration and angular acceleration of

@@ -588,6 +588,7 @@ int launch_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd,
 // becomes live), FP64 or FP32 form; *input = the record buffer the pass read
 int launch_step(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, int form, bool gravity_on,
                 V3 g, double thr2, int32_t step_tag, Core** input);
+int finish_step(xdem_ctx* c, int32_t trig_out, Core** input);  // after an integrating pass (contact_sphere.hip)
 int alloc_walls(xdem_ctx* c, int nw);
 // mesh candidates + history carry-over (poly: the polyhedron candidates of the particles' vertices, edges
 // and faces, built by launch_poly_mesh_carry)

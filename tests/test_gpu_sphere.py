@@ -680,3 +680,38 @@ def test_simulation_state(gpu_ok, case):
     print(f"{case}: {st['n_interactions']} interactions, {st['n_active']} active, min dn {st['min_dn']:.6g}")
     assert st["n_interactions"] == tot and st["n_active"] == act and act > 0
     assert abs(st["min_dn"] - min_dn) <= 1e-12 and min_dn < 0
+
+
+@pytest.mark.parametrize("n", [1, 33, 1000, 36001, 45001, 64001])
+def test_step_lane_splits_match_oracle(gpu_ok, n):
+    """Both sides of the sizes at which a step changes between eight, four and one lane per particle, and the edges of
+    their blocks (32 and 64 particles): positions, velocities, spins, forces, moments and friction after engine and
+    operator steps equal the oracle's bit for bit; the FP32-force form's forces within its stated 1e-5."""
+    def fresh():
+        side = max(4, int(np.ceil((n / 1.5) ** (1.0 / 3.0))))
+        edge = 0.98 * (side - 1) + 0.96
+        w = inputs.deposition(n=n, spacing=0.98, seed=n, start=0.48, box=(edge, edge, 2 * edge + 2))
+        rng = np.random.default_rng(n)
+        for k in ("vx", "vy", "vz", "vrotx", "vroty", "vrotz"):
+            w.particles[k] = rng.normal(0, 0.3, n)
+        return w
+    w = fresh()
+    s = SphereSim(w)
+    s.first_iteration()
+    s.run(5, poll=3)
+    s.step()
+    o = po.Oracle(w.particles, w.domain, w.walls)
+    o.first_iteration(scheme(w))
+    o.run_steps(scheme(w), 6)
+    a, b = by_id(s.ctx.download()), by_id(o.particles())
+    for k in ("rx", "ry", "rz", "vx", "vy", "vz", "qw", "qx", "qy", "qz", "vrotx", "vroty", "vrotz", "fx", "fy", "fz",
+              "momx", "momy", "momz"):
+        assert np.array_equal(a[k], b[k]), k
+    ka, fa = interaction_table(*s.ctx.interactions())
+    kb, fb = interaction_table(*o.interactions()[:4])
+    assert np.array_equal(ka, kb) and np.array_equal(fa, fb)
+    f = SphereSim(fresh(), form=native.XDEM_FORM_FP32)
+    f.first_iteration()
+    f.run(6, poll=3)
+    c = by_id(f.ctx.download())
+    assert rel_err(force(c), force(a), 9.81) <= 1e-5
