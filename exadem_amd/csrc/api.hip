@@ -1003,12 +1003,12 @@ int xdem_run_steps(xdem_ctx* c, const xdem_scheme* s, int64_t nsteps, xdem_run_s
   }
   XDEM_HIP(c, hipMemsetAsync(c->d_flags, 0, 4 * sizeof(int32_t), c->stream));
   c->trig_slot = 0;
-  // spheres run a step as one kernel (force pass + kick + next prolog into the other record buffer,
-  // launch_step) between a chain-start prolog and the last step of the run, which keeps the separate
-  // kernels so that the run ends in the same state (pending kick flushed) as the operator sequence.
-  // (Polyhedra keep separate kernels: an integrating gather that also recomputes the vertices measured
-  // no faster than the separate vertex pass.)
-  const bool fuse = c->nshapes == 0;
+  // A step inside a chain runs as an integrating force pass: spheres in one kernel (force pass + kick + next prolog into
+  // the other record buffer, launch_step), polyhedra in two (feature pass, integrating gather with the vertices, in
+  // place). A chain starts with a prolog of its own, and the last step of the run keeps the separate kernels, so that
+  // the run ends in the same state (pending kick flushed) as the operator sequence. Recorded polyhedron passes
+  // (xdem_set_contact_record) are not integrating.
+  const bool fuse = c->nshapes == 0 || !c->record_cs;
   std::vector<Core*> input(poll);   // record buffer read by the integrating pass of each step of a chunk
   std::vector<double> times(poll + 1);  // physical time at the start of each step of a chunk
   bool chain = false;               // the live records hold the prolog of the next step
@@ -1056,9 +1056,12 @@ int xdem_run_steps(xdem_ctx* c, const xdem_scheme* s, int64_t nsteps, xdem_run_s
       }
       if (timed && (rc = record_timer(c, 1, true))) return rc;
       if (fuse && step + 1 < nsteps) {
-        if ((rc = launch_step(c, cp, cpd, s->dt, s->form, s->gravity_on != 0, g, thr * thr, (int32_t)step,
-                              &input[step - done])))
+        if (poly) {
+          if ((rc = poly_force(c, cp, cpd, s->dt, true, s->gravity_on != 0, g, true, (int32_t)step, thr * thr))) return rc;
+        } else if ((rc = launch_step(c, cp, cpd, s->dt, s->form, s->gravity_on != 0, g, thr * thr, (int32_t)step,
+                                     &input[step - done]))) {
           return rc;
+        }
         chain = true;
         c->pending_kick = false;
       } else {

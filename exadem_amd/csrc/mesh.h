@@ -246,28 +246,5 @@ __device__ inline void mesh_add_at(const MeshTerms& t, uint2 mi, V3& F, V3& M) {
     }
   }
 }
-// The same sums with four loads in flight per batch and no pipelining across batches (fewer registers:
-// the polyhedra gather, where the pipelined form lowers occupancy).
-__device__ inline void mesh_add(const MeshTerms& t, int64_t x, V3& F, V3& M) {
-  const uint2 mi = t.idx[x];
-  const uint32_t c = mi.y;
-  const double2* p = reinterpret_cast<const double2*>(t.terms) + (int64_t)mi.x * 3;
-  for (uint32_t k0 = 0; k0 < c; k0 += 4) {
-    double2 r[4][3] = {};
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-      if (k0 + q < c) {
-        r[q][0] = p[(k0 + q) * 3];
-        r[q][1] = p[(k0 + q) * 3 + 1];
-        r[q][2] = p[(k0 + q) * 3 + 2];
-      }
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-      if (k0 + q < c) {
-        F = F + V3{r[q][0].x, r[q][0].y, r[q][1].x};
-        M = M + V3{r[q][1].y, r[q][2].x, r[q][2].y};
-      }
-  }
-}
 
 }  // namespace xdem

@@ -13,14 +13,15 @@
 //
 // Contact pass without atomics: one thread per feature evaluates it and writes its terms of the owner
 // force, owner moment and partner moment (the partner's force term is the exact negation). A second
-// kernel walks, per particle and in stream order, its entries (each slot holds its pair's feature range,
-// the owner slot's for a partner entry), forms each pair's subtotal over the features in list order,
-// adds it, then the vertex-wall contacts, then finishes force_to_accel and the angular acceleration.
+// kernel sums each particle's entries in stream order (each slot holds its pair's feature range, the owner
+// slot's for a partner entry), each pair's subtotal formed over the features in list order, then the
+// vertex-wall contacts, then finishes force_to_accel and the angular acceleration, or the particle's whole step.
 #include <algorithm>
 #include <unordered_map>
 
 #include "contact_law.h"
 #include "mesh.h"
+#include "step.h"
 
 namespace xdem {
 
@@ -1305,6 +1306,10 @@ struct PolyForceArgs {
   int32_t* flags;
   int32_t step_tag;
   MeshTerms mt;  // terms of the mesh contacts, evaluated by k_poly_mesh_pass just before (ncand = 0: none)
+  // integrating gather: where the new vertices go, kick dt/2 of the finished step, squared displacement threshold
+  d4* vtx_out;
+  double kdt_2;
+  double thr2;
 };
 
 __device__ inline bool poly_guard(const PolyForceArgs& a) {
@@ -1433,179 +1438,313 @@ __global__ __launch_bounds__(128) void k_poly_feat(PolyForceArgs a) {
   }
 }
 
-struct Q4p {
-  double w, x, y, z;
-};
-__device__ inline V3 angular_accel_p(const d4& q, V3 mom, V3 vrot, V3 I) {
-  const d4 qi{q.x, -q.y, -q.z, -q.w};
-  const V3 om = qrot4(qi, vrot);
-  const V3 M = qrot4(qi, mom);
-  const V3 dom{(M.x - (I.z - I.y) * om.y * om.z) / I.x, (M.y - (I.x - I.z) * om.z * om.x) / I.y,
-               (M.z - (I.y - I.x) * om.x * om.y) / I.z};
-  return qrot4(q, dom);
+// The particles' sums, L lanes per particle (256 / L particles per block). A lane takes one list entry of a round of L: it
+// scans the flags of its pair's features and forms the pair's subtotal over the features in contact in feature order, as
+// the owner's pass forms it. The subtotals go through LDS to two threads per particle (force, moment), which add them in
+// list order; the vertex-wall contacts are rounds of the same kind, one candidate (set bit of the mask) per lane. Lanes
+// without an entry write -0.0, which adds nothing to any value, so every sum has the terms and the order of one thread
+// walking the list. Then the two threads finish the particle: force_to_accel and the angular acceleration, or, INTEG,
+// its epilog kick and the prolog of the next step (kick_prolog's linear part on the one, its rotation on the other, in
+// another wavefront), in place, since no other block reads these records; after that the lanes compute the world
+// vertices of the new pose and test their displacement (flags[0] raised for the next step's pass).
+//
+// With one thread per particle, which walked its entries and their contacts one after the other, the pass lasted as long
+// as the longest such walk (57 us at 20k polyhedra in a dense moving bed), and the prolog with the vertices was a pass
+// of its own (31 us at 200k). Engine step: 64.8 -> 39.2 us at 20k moving, 94.0 -> 73.1 us at 200k at rest.
+__device__ inline d4 rec_d4(const uint4* p) {  // LDS rows of records are 16-byte aligned
+  d4 v;
+  __builtin_memcpy(&v, p, sizeof(d4));
+  return v;
 }
-
-template <bool FUSED, bool KR, bool GUARD>
-__global__ __launch_bounds__(256) void k_poly_gather(PolyForceArgs a) {
-  // the stall decision was taken by k_poly_feat of the same step
-  if (GUARD && a.flags[1]) return;
+template <int L, bool FUSED, bool KR, bool GUARD, bool INTEG>
+__global__ __launch_bounds__(256, 4) void k_poly_gather(PolyForceArgs a) {
+  // the stall decision was taken by k_poly_feat of the same step; the flag is read with the first loads and tested
+  // before the first store
+  const bool stop = GUARD && a.flags[1];
+  constexpr int NP = 256 / L, ROW = NP + 8, M0 = NP < 64 ? 64 : NP;
+  constexpr int NV = XDEM_MAX_SHAPE_VERTICES / L;  // vertices per lane
+  constexpr int CH = NP * 8 / 256;                 // 16-byte chunks of the block's records per thread
+  __shared__ double con[6][L * ROW];
+  __shared__ uint4 rec[NP * 8];  // the block's records
+  __shared__ double aux[FUSED ? (INTEG ? 10 : 3) : 1][NP];  // inertia; rebuild position and orientation
+  const int tid = threadIdx.x, p = tid / L, sub = tid % L;
   // XCD-aware block order (partner contributions are read through the owner slots' feature ranges)
-  const int64_t b0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x;
-  // the block's 256 records, staged in LDS with coalesced 16-byte copies: the mass is read from there
-  // before the list walk and the rest of the record after it, without holding it in registers
-  __shared__ Core tile[256];
-  stage_tile(tile, a.s.core, b0, a.n);
-  __syncthreads();
-  const int64_t x = b0 + threadIdx.x;
-  if (x >= a.n) return;
+  const int64_t b0 = xcd_block(blockIdx.x, gridDim.x) * NP;
   const PState& s = a.s;
-  const double mx = tile[threadIdx.x].vm.w;
-  V3 F, M;
-  if (FUSED) {
-    F = {0.0, 0.0, 0.0};
-    M = {0.0, 0.0, 0.0};
-    if (a.gravity_on) F = {F.x + a.grav.x * mx, F.y + a.grav.y * mx, F.z + a.grav.z * mx};
-  } else {
-    F = {s.ax[x], s.ay[x], s.az[x]};
-    M = {s.mx[x], s.my[x], s.mz[x]};
+  const int64_t x = b0 + p;
+  const bool in = x < a.n;
+  const int64_t xc = in ? x : a.n - 1;
+  const uint32_t cnt = in ? a.nl.cnt[xc] : 0u;
+  const uint64_t base = a.nl.base[xc >> 6] + (uint64_t)(xc & 63);
+  const uint32_t kmax = a.nl.kmax[b0 >> 6];
+  uint4 chunk[CH];
+#pragma unroll
+  for (int q = 0; q < CH; q++) {
+    const int64_t at = b0 + ((tid + 256 * q) >> 3);
+    chunk[q] = ((const uint4*)(s.core + (at < a.n ? at : a.n - 1)))[tid & 7];
   }
-  const uint32_t cnt = a.nl.cnt[x];
-  const uint64_t b = a.nl.base[x >> 6] + (uint64_t)(x & 63);
-  // per entry, the pair subtotal in feature order (as the owner's pass forms it), then the sum; the
-  // word and feature range of entry k+1 are loaded while entry k is summed
-  uint32_t wd_n = 0;
-  uint2 fr_n{0u, 0u};
-  if (cnt > 0) {
-    wd_n = a.nl.word[b];
-    fr_n = a.frange[b];
-  }
-  for (uint32_t k = 0; k < cnt; k++) {
-    const uint64_t sl = b + (uint64_t)k * kWave;
-    const uint32_t wd = wd_n;
-    const uint2 fr = fr_n;
-    if (k + 1 < cnt) {
-      wd_n = a.nl.word[sl + kWave];
-      fr_n = a.frange[sl + kWave];
+  uint64_t mask = 0;
+  if (a.nw > 0 && in) mask = a.pw.mask[xc];
+  // the lane's vertices of the particle's shape, for the new vertices
+  const xdem_shape& sh = a.shapes[s.type[xc]];
+  V3 body[NV];
+  int nv = 0;
+  if (INTEG) {
+    nv = sh.nv;
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+      const int k = sub + q * L;  // (the shape record has room for all eight)
+      body[q] = V3{sh.vertices[k][0], sh.vertices[k][1], sh.vertices[k][2]};
     }
-    const bool own = (wd & kOwnerBit) != 0;
-    if (fr.x == 0xffffffffu) continue;
-    V3 Fp{0, 0, 0}, Mp{0, 0, 0};
-    const uint64_t f0 = fr.x, f1 = (uint64_t)fr.x + fr.y;
-    // the pair's contact flags as aligned 32-bit words, four words (16 flags) in flight at a time (the
-    // flag array has at least 4096 bytes of padding), then its features in contact in feature order
-    const uint32_t* __restrict__ cw = reinterpret_cast<const uint32_t*>(a.contact);
-    const uint64_t wend = (f1 + 3) >> 2;
-    for (uint64_t w0 = f0 >> 2; w0 < wend; w0 += 4) {
-      uint32_t v[4];
+  }
+  // the first entry's feature range and word (~0u: no entry, or no owner entry); each later one a round ahead
+  uint2 range{0xffffffffu, 0u};
+  uint32_t wd = 0;
+  if ((uint32_t)sub < cnt) {
+    range = a.frange[base + (uint64_t)sub * kWave];
+    wd = a.nl.word[base + (uint64_t)sub * kWave];
+  }
+  // summing threads
+  const bool fr = tid < NP && b0 + tid < a.n;
+  const bool mo = tid >= M0 && tid < M0 + NP && b0 + tid - M0 < a.n;
+  const int sp = mo ? tid - M0 : (fr ? tid : 0), c0 = mo ? 3 : 0;
+  const int64_t xi = b0 + sp;
+  V3 S{0.0, 0.0, 0.0};
+  if (!FUSED && fr) S = {s.ax[xi], s.ay[xi], s.az[xi]};
+  if (!FUSED && mo) S = {s.mx[xi], s.my[xi], s.mz[xi]};
+  if (GUARD && stop) return;
+  if (FUSED) {
 #pragma unroll
-      for (int q = 0; q < 4; q++) v[q] = w0 + q < wend ? cw[w0 + q] : 0u;
+    for (int q = 0; q < ((INTEG ? 10 : 3) * NP + 255) / 256; q++) {
+      const int c = (tid + 256 * q) / NP, i = tid & (NP - 1);
+      const int64_t at = b0 + i < a.n ? b0 + i : a.n - 1;
+      if (c == 0) aux[0][i] = s.ix[at];
+      if (c == 1) aux[1][i] = s.iy[at];
+      if (c == 2) aux[2][i] = s.iz[at];
+      if (INTEG && c == 3) aux[3][i] = s.bx[at];
+      if (INTEG && c == 4) aux[4][i] = s.by[at];
+      if (INTEG && c == 5) aux[5][i] = s.bz[at];
+      if (INTEG && c >= 6 && c < 10) aux[c][i] = reinterpret_cast<const double*>(s.bq + at)[c - 6];
+    }
+  }
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        // the word's features in contact; for each half word in which any lane of the wavefront has one,
-        // the two features' terms are loaded together (a position without a hit reads row 0, which exists
-        // whenever some feature is in contact, and discards it), then added in feature order
-        uint32_t hits = 0;
+  for (int q = 0; q < CH; q++) rec[tid + 256 * q] = chunk[q];
+  const uint32_t rounds = (kmax + L - 1) / L;
+  auto begin = [&]() {  // after the first barrier: the records are staged
+    if (FUSED && fr && a.gravity_on) {
+      const double m = rec_d4(rec + sp * 8 + 2).w;
+      S = {0.0 + a.grav.x * m, 0.0 + a.grav.y * m, 0.0 + a.grav.z * m};
+    }
+  };
+  auto add_round = [&]() {
+    if (fr || mo) {
 #pragma unroll
-        for (int byte = 0; byte < 4; byte++) {
-          const uint64_t f = ((w0 + q) << 2) + byte;
-          if (((v[q] >> (8 * byte)) & 0xffu) != 0u && f >= f0 && f < f1) hits |= 1u << byte;
-        }
+      for (int u = 0; u < L; u++)
+        S = S + V3{con[c0][u * ROW + sp], con[c0 + 1][u * ROW + sp], con[c0 + 2][u * ROW + sp]};
+    }
+  };
+  auto put = [&](V3 f, V3 m) {
+    const int o = sub * ROW + p;
+    con[0][o] = f.x; con[1][o] = f.y; con[2][o] = f.z;
+    con[3][o] = m.x; con[4][o] = m.y; con[5][o] = m.z;
+  };
+  if (rounds == 0) {
+    __syncthreads();
+    begin();
+  }
+  for (uint32_t r = 0; r < rounds; r++) {
+    const uint32_t k = r * L + (uint32_t)sub;
+    V3 Fp{-0.0, -0.0, -0.0}, Mp{-0.0, -0.0, -0.0};
+    {
+      const uint2 cur = range;
+      const bool own = (wd & kOwnerBit) != 0;
+      range.x = 0xffffffffu;
+      if (k + L < cnt) {
+        range = a.frange[base + (uint64_t)(k + L) * kWave];
+        wd = a.nl.word[base + (uint64_t)(k + L) * kWave];
+      }
+      if (cur.x != 0xffffffffu) {
+        Fp = V3{0.0, 0.0, 0.0};
+        Mp = V3{0.0, 0.0, 0.0};
+        const uint64_t f0 = cur.x, f1 = (uint64_t)cur.x + cur.y;
+        // the pair's contact flags as aligned 32-bit words, four words (16 flags) in flight at a time (the flag
+        // array has at least 4096 bytes of padding), then its features in contact in feature order, two at a time
+        const uint32_t* __restrict__ cw = reinterpret_cast<const uint32_t*>(a.contact);
+        const uint64_t wend = (f1 + 3) >> 2;
+        for (uint64_t w0 = f0 >> 2; w0 < wend; w0 += 4) {
+          uint32_t v[4], hits = 0;
 #pragma unroll
-        for (int h = 0; h < 4; h += 2) {
-          const uint32_t hh = (hits >> h) & 3u;
-          if (__builtin_amdgcn_ballot_w64(hh != 0u) == 0ull) continue;
-          V3 tf[2], tm[2];
+          for (int q = 0; q < 4; q++) v[q] = w0 + q < wend ? cw[w0 + q] : 0u;
 #pragma unroll
-          for (int e = 0; e < 2; e++) {
-            const uint64_t f = ((hh >> e) & 1u) ? ((w0 + q) << 2) + h + e : 0u;
-            const double* pr = a.contrib + 9 * f;
-            tf[e] = V3{pr[0], pr[1], pr[2]};
-            tm[e] = own ? V3{pr[3], pr[4], pr[5]} : V3{pr[6], pr[7], pr[8]};
-          }
-#pragma unroll
-          for (int e = 0; e < 2; e++) {
-            if (!((hh >> e) & 1u)) continue;
-            if (own) Fp = Fp + tf[e];
-            else Fp = Fp + V3{-tf[e].x, -tf[e].y, -tf[e].z};
-            Mp = Mp + tm[e];
+          for (int q = 0; q < 4; q++)
+            hits |= ((v[q] & 1u) | ((v[q] >> 7) & 2u) | ((v[q] >> 14) & 4u) | ((v[q] >> 21) & 8u)) << (4 * q);
+          const uint64_t g0 = w0 << 2;
+          if (f0 > g0) hits &= 0xffffu << (uint32_t)(f0 - g0);
+          if (f1 < g0 + 16) hits &= 0xffffu >> (uint32_t)(g0 + 16 - f1);
+          while (hits) {
+            const uint32_t i0 = (uint32_t)__builtin_ctz(hits);
+            hits &= hits - 1u;
+            const bool two = hits != 0u;
+            const uint32_t i1 = two ? (uint32_t)__builtin_ctz(hits) : i0;
+            hits &= hits - 1u;
+            const double *p0 = a.contrib + 9 * (g0 + i0), *p1 = a.contrib + 9 * (g0 + i1);
+            const int mo_ = own ? 3 : 6;
+            const V3 ta{p0[0], p0[1], p0[2]}, ma{p0[mo_], p0[mo_ + 1], p0[mo_ + 2]};
+            const V3 tb{p1[0], p1[1], p1[2]}, mb{p1[mo_], p1[mo_ + 1], p1[mo_ + 2]};
+            Fp = Fp + (own ? ta : -ta);
+            Mp = Mp + ma;
+            if (two) {
+              Fp = Fp + (own ? tb : -tb);
+              Mp = Mp + mb;
+            }
           }
         }
       }
     }
-    F = F + Fp;
-    M = M + Mp;
+    if (r > 0) __syncthreads();  // the previous round's terms are added
+    put(Fp, Mp);
+    __syncthreads();
+    if (r == 0) begin();
+    add_round();
   }
-  // the record's fields are read from the tile where they are used below
-  const Core& cx = tile[threadIdx.x];
   if (a.nw > 0) {
-    const xdem_shape& sh = a.shapes[s.type[x]];
-    const double r = sh.minkowski * cx.w.w;
-    const uint64_t mask = a.pw.mask[x];
-    const V3 rx{cx.xr.x, cx.xr.y, cx.xr.z}, vx{cx.vm.x, cx.vm.y, cx.vm.z}, wx{cx.w.x, cx.w.y, cx.w.z};
-    for (int w = 0; w < a.nw; w++)
-      for (int k = 0; k < sh.nv; k++) {
-        const int bit = w * XDEM_MAX_SHAPE_VERTICES + k;
-        if (!((mask >> bit) & 1ull)) continue;
+    while (__syncthreads_or(mask != 0)) {
+      V3 Fw{-0.0, -0.0, -0.0}, Mw{-0.0, -0.0, -0.0};
+      uint64_t t = mask;
+      for (int q = 0; q < sub; q++) t &= t - 1;
+      if (t) {
+        // vertex k of the particle against wall w
+        const int bit = __builtin_ctzll(t);
+        const int w = bit / XDEM_MAX_SHAPE_VERTICES, k = bit % XDEM_MAX_SHAPE_VERTICES;
+        const d4 xr = rec_d4(rec + p * 8), vm = rec_d4(rec + p * 8 + 2), om = rec_d4(rec + p * 8 + 4);
+        const double rm = sh.minkowski * om.w;
+        const V3 rx{xr.x, xr.y, xr.z};
         const int64_t j = (int64_t)bit * a.wstride + x;
         const d4 v4 = a.vtx[x * XDEM_MAX_SHAPE_VERTICES + k];
-        const V3 p{v4.x, v4.y, v4.z};
         const Surface& sf = a.walls[w];
         double dn;
         V3 nrm, cpos;
-        if (!driver_detect(sf, p, r, dn, nrm, cpos)) {
+        if (!driver_detect(sf, V3{v4.x, v4.y, v4.z}, rm, dn, nrm, cpos)) {
           a.pw.hx[j] = 0.0; a.pw.hy[j] = 0.0; a.pw.hz[j] = 0.0;
           a.pw.mhx[j] = 0.0; a.pw.mhy[j] = 0.0; a.pw.mhz[j] = 0.0;
-          if (a.wstate) {
+          if (!INTEG && a.wstate) {
             double* rc = a.wstate + (uint64_t)kCStateLen * j;
 #pragma unroll
             for (int q = 0; q < kCStateLen; q++) rc[q] = 0.0;
           }
-          continue;
-        }
-        V3 ft{a.pw.hx[j], a.pw.hy[j], a.pw.hz[j]};
-        V3 mint{0.0, 0.0, 0.0};
-        if (KR) mint = {a.pw.mhx[j], a.pw.mhy[j], a.pw.mhz[j]};
-        const V3 f = hooke_force<KR>(dn, nrm, a.dt, a.cpd, mx, ft, mint, cpos, rx, vx, wx, sf.center, sf.vel, sf.vrot);
-        if (a.wstate) {
-          const V3 fnv = f - ft;
-          const double rec[kCStateLen] = {dn,   cpos.x, cpos.y, cpos.z, fnv.x, fnv.y, fnv.z, ft.x,
-                                          ft.y, ft.z,   rx.x,   rx.y,   rx.z,   0.0,   0.0,   0.0};
-          double* rc = a.wstate + (uint64_t)kCStateLen * j;
+        } else {
+          V3 ft{a.pw.hx[j], a.pw.hy[j], a.pw.hz[j]};
+          V3 mint{0.0, 0.0, 0.0};
+          if (KR) mint = {a.pw.mhx[j], a.pw.mhy[j], a.pw.mhz[j]};
+          const V3 f = hooke_force<KR>(dn, nrm, a.dt, a.cpd, vm.w, ft, mint, cpos, rx, V3{vm.x, vm.y, vm.z},
+                                       V3{om.x, om.y, om.z}, sf.center, sf.vel, sf.vrot);
+          if (!INTEG && a.wstate) {
+            const V3 fnv = f - ft;
+            const double row[kCStateLen] = {dn,   cpos.x, cpos.y, cpos.z, fnv.x, fnv.y, fnv.z, ft.x,
+                                            ft.y, ft.z,   rx.x,   rx.y,   rx.z,  0.0,   0.0,   0.0};
+            double* rc = a.wstate + (uint64_t)kCStateLen * j;
 #pragma unroll
-          for (int q = 0; q < kCStateLen; q++) rc[q] = rec[q];
+            for (int q = 0; q < kCStateLen; q++) rc[q] = row[q];
+          }
+          a.pw.hx[j] = ft.x; a.pw.hy[j] = ft.y; a.pw.hz[j] = ft.z;
+          if (KR) {
+            a.pw.mhx[j] = mint.x; a.pw.mhy[j] = mint.y; a.pw.mhz[j] = mint.z;
+          }
+          Fw = f;
+          Mw = cross(cpos - rx, f) + mint;
         }
-        a.pw.hx[j] = ft.x; a.pw.hy[j] = ft.y; a.pw.hz[j] = ft.z;
-        if (KR) {
-          a.pw.mhx[j] = mint.x; a.pw.mhy[j] = mint.y; a.pw.mhz[j] = mint.z;
-        }
-        F = F + f;
-        M = M + (cross(cpos - rx, f) + mint);
       }
+      put(Fw, Mw);  // (the loop's barrier: the previous terms are added)
+      __syncthreads();
+      add_round();
+      for (int q = 0; q < L; q++) mask &= mask - 1;
+    }
   }
-  if (a.mt.ncand) mesh_add(a.mt, x, F, M);
-  if (FUSED) {
-    s.ax[x] = F.x / mx;
-    s.ay[x] = F.y / mx;
-    s.az[x] = F.z / mx;
-    s.mx[x] = M.x;
-    s.my[x] = M.y;
-    s.mz[x] = M.z;
-    const V3 al = angular_accel_p(cx.q, M, V3{cx.w.x, cx.w.y, cx.w.z}, V3{s.ix[x], s.iy[x], s.iz[x]});
-    s.alx[x] = al.x;
-    s.aly[x] = al.y;
-    s.alz[x] = al.z;
-  } else {
-    s.ax[x] = F.x;
-    s.ay[x] = F.y;
-    s.az[x] = F.z;
-    s.mx[x] = M.x;
-    s.my[x] = M.y;
-    s.mz[x] = M.z;
+  if (a.mt.ncand && (fr || mo)) {
+    const uint2 mi = a.mt.idx[xi];
+    const double* t = a.mt.terms + (int64_t)mi.x * 6 + c0;
+    for (uint32_t u = 0; u < mi.y; u++) S = S + V3{t[6 * u], t[6 * u + 1], t[6 * u + 2]};
+  }
+  uint4* row = rec + sp * 8 + (mo ? 4 : 0);  // position and velocity, or spin and orientation
+  if (fr) {
+    if (!FUSED) {
+      s.ax[xi] = S.x;
+      s.ay[xi] = S.y;
+      s.az[xi] = S.z;
+    } else {
+      d4 xr = rec_d4(row), vm = rec_d4(row + 2);
+      const V3 acc{S.x / vm.w, S.y / vm.w, S.z / vm.w};
+      if (!INTEG) {
+        s.ax[xi] = acc.x;
+        s.ay[xi] = acc.y;
+        s.az[xi] = acc.z;
+      } else {
+        d4 w{}, qq{1.0, 0.0, 0.0, 0.0};
+        kick_prolog<true>(xr, vm, w, qq, acc.x, acc.y, acc.z, 0.0, 0.0, 0.0, a.dt, a.kdt_2);
+        __builtin_memcpy(row, &xr, sizeof(d4));
+        __builtin_memcpy(row + 2, &vm, sizeof(d4));
+      }
+    }
+  } else if (mo) {
+    if (!INTEG) {
+      s.mx[xi] = S.x;
+      s.my[xi] = S.y;
+      s.mz[xi] = S.z;
+    }
+    if (FUSED) {
+      d4 w = rec_d4(row), qq = rec_d4(row + 2);
+      const V3 al = angular_accel(Q4{qq.x, qq.y, qq.z, qq.w}, S, V3{w.x, w.y, w.z},
+                                  V3{aux[0][sp], aux[1][sp], aux[2][sp]});
+      if (!INTEG) {
+        s.alx[xi] = al.x;
+        s.aly[xi] = al.y;
+        s.alz[xi] = al.z;
+      } else {
+        d4 xr{}, vm{};
+        kick_prolog<true>(xr, vm, w, qq, 0.0, 0.0, 0.0, al.x, al.y, al.z, a.dt, a.kdt_2);
+        __builtin_memcpy(row, &w, sizeof(d4));
+        __builtin_memcpy(row + 2, &qq, sizeof(d4));
+      }
+    }
+  }
+  if (INTEG) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < CH; q++) {
+      const int64_t at = b0 + ((tid + 256 * q) >> 3);
+      if (at < a.n) ((uint4*)(s.core + at))[tid & 7] = rec[tid + 256 * q];
+    }
+    if (!in) return;
+    // get_vertex of the new pose and of the pose at the last rebuild
+    const d4 xr = rec_d4(rec + p * 8), w = rec_d4(rec + p * 8 + 4), qn = rec_d4(rec + p * 8 + 6);
+    const V3 r0{aux[3][p], aux[4][p], aux[5][p]};
+    const d4 q0{aux[6][p], aux[7][p], aux[8][p], aux[9][p]};
+    bool moved = false;
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+      const int k = sub + q * L;
+      if (k >= nv) continue;
+      const V3 hv = w.w * body[q];
+      const V3 v = V3{xr.x, xr.y, xr.z} + qrot4(qn, hv);
+      a.vtx_out[x * XDEM_MAX_SHAPE_VERTICES + k] = {v.x, v.y, v.z, 0.0};
+      const V3 d = v - (r0 + qrot4(q0, hv));
+      if (dot(d, d) >= a.thr2) moved = true;
+    }
+    if (moved) a.flags[0] = 1;
   }
 }
 
+// Lanes per particle of the gather (us per step of the engine, eight / four / two lanes, a moving bed and at 200,000 the
+// bed at rest): 2,000: 30.3 / 32.1 / 39.5; 20,000: 39.2 / 39.5 / 45.1; 60,000: 72.0 / 66.5 / 71.7; 200,000: 84.0 / 73.1 /
+// 73.1. A block's life is its chain of dependent loads and barriers: while all blocks of 32 particles are resident at once
+// (four per CU at 118 registers, 256 CUs) the shortest chain wins, beyond that the fewest blocks.
+constexpr int64_t kGather8Max = 4 * 256 * 32;
+inline int gather_lanes(int64_t n) { return n <= kGather8Max ? 8 : 4; }
+
 int poly_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, bool fused, bool gravity_on,
-               V3 g, bool guarded, int32_t step_tag) {
+               V3 g, bool guarded, int32_t step_tag, double integ_thr2) {
+  const bool integ = integ_thr2 >= 0;  // an engine step (fused, guarded): the gather integrates
+
   if (!c->pl_valid || !c->hist_ready || c->pl_epoch != c->nl_epoch)
     return set_err(c, XDEM_ERR_STATE, "contact_polyhedron: run nbh_polyhedron after chunk_neighbors_contact");
   if (c->pl_class_epoch != c->nl_epoch)
@@ -1638,6 +1777,9 @@ int poly_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, d
   a.gravity_on = gravity_on ? 1 : 0;
   a.flags = c->d_flags;
   a.step_tag = step_tag;
+  a.vtx_out = c->vtx;
+  a.kdt_2 = dt * 0.5;
+  a.thr2 = integ_thr2;
   int rc;
   if (c->record_cs) {
     if (a.pl.nfeat > c->cap_cstate) {
@@ -1686,29 +1828,36 @@ int poly_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, d
     }
     XDEM_HIP(c, hipGetLastError());
   }
-  const dim3 gp(grid_blocks(std::max<int64_t>(a.norder, 1), 128)), bp(128), gg(grid_blocks(a.n, 256)),
-      bg(256);
+  const dim3 gp(grid_blocks(std::max<int64_t>(a.norder, 1), 128)), bp(128), bg(256);
   const bool kr = c->kr_used;
+  const int lanes = gather_lanes(a.n);
+  const dim3 gg(grid_blocks(a.n, 256 / lanes));
 #define PAIRS(KRV, G) hipLaunchKernelGGL((k_poly_feat<KRV, G>), gp, bp, 0, c->stream, a)
-#define GATHER(F, KRV, G) hipLaunchKernelGGL((k_poly_gather<F, KRV, G>), gg, bg, 0, c->stream, a)
+#define GATHER(LN, F, KRV, G, I) hipLaunchKernelGGL((k_poly_gather<LN, F, KRV, G, I>), gg, bg, 0, c->stream, a)
+#define GATHER_KR(F, G, I)                            \
+  do {                                                \
+    if (lanes == 8 && kr) GATHER(8, F, true, G, I);   \
+    else if (lanes == 8) GATHER(8, F, false, G, I);   \
+    else if (kr) GATHER(4, F, true, G, I);             \
+    else GATHER(4, F, false, G, I);                    \
+  } while (0)
   if (kr) {
     if (guarded) PAIRS(true, true); else PAIRS(true, false);
   } else {
     if (guarded) PAIRS(false, true); else PAIRS(false, false);
   }
-  if (fused) {
-    if (kr) { if (guarded) GATHER(true, true, true); else GATHER(true, true, false); }
-    else { if (guarded) GATHER(true, false, true); else GATHER(true, false, false); }
-  } else {
-    if (kr) { if (guarded) GATHER(false, true, true); else GATHER(false, true, false); }
-    else { if (guarded) GATHER(false, false, true); else GATHER(false, false, false); }
-  }
+  if (integ) GATHER_KR(true, true, true);
+  else if (fused && guarded) GATHER_KR(true, true, false);
+  else if (fused) GATHER_KR(true, false, false);
+  else GATHER_KR(false, false, false);
 #undef PAIRS
 #undef GATHER
+#undef GATHER_KR
   XDEM_HIP(c, hipGetLastError());
   c->cs_valid = c->record_cs;
   c->cs_epoch = c->nl_epoch;
   c->poly_pass_epoch = c->nl_epoch;
+  if (integ) c->cells_valid = false;  // positions moved: the binning no longer matches them
   return XDEM_OK;
 }
 

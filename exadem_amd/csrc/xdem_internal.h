@@ -620,8 +620,10 @@ int launch_prolog_verts(xdem_ctx* c, double dt, bool with_kick, double kick_dt, 
 int poly_nbh(xdem_ctx* c, double rcut_inc);
 // classify_interactions of polyhedra: the feature waves by type (forder, fwave_start, fwave_size)
 int poly_classify(xdem_ctx* c);
+// integ_thr2 >= 0: a step of the engine, whose gather integrates the particles (kick, next prolog, vertices) and raises
+// the rebuild trigger where a vertex moved by sqrt(integ_thr2)
 int poly_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, double dt, bool fused, bool gravity_on,
-               V3 g, bool guarded, int32_t step_tag);
+               V3 g, bool guarded, int32_t step_tag, double integ_thr2 = -1.0);
 // interaction counts of the polyhedron lists for simulation_state: total, active, smallest dn; block
 // partials in the library's buffer (fixed = null) or in the fixed buffer of fixed_cap doubles
 int poly_sim_counts(xdem_ctx* c, double* tot, double* act, double* min_dn, double* fixed, int64_t fixed_cap);
