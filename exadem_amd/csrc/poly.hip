@@ -198,10 +198,10 @@ struct FaceFrame {
   double q1[XDEM_MAX_FACE_VERTICES], q2[XDEM_MAX_FACE_VERTICES];
   int nf;
 };
-__device__ inline FaceFrame face_frame(const Verts& vj, const xdem_shape& shj, int face) {
+// vj: the body's vertices by index; f: the face's nf vertex indices
+template <class V, class I>
+__device__ inline FaceFrame face_frame(const V& vj, const I* f, int nf) {
   FaceFrame fr;
-  const int nf = shj.face_size[face];
-  const int* f = shj.faces[face];
   const V3 va = vj[f[0]];
   const V3 vb = vj[f[1]];
   const V3 vc = vj[f[nf - 1]];
@@ -436,7 +436,7 @@ __device__ inline void for_each_feature(const PolyNbhArgs& a, int64_t x, uint32_
   if (gate_a) {
     const double lim = ra + rb + rv;
     for (int j = 0; j < sb.nf; j++) {
-      const FaceFrame fr = face_frame(vb, sb, j);
+      const FaceFrame fr = face_frame(vb, sb.faces[j], sb.face_size[j]);
       for (int i = 0; i < sa.nv; i++)
         if (((gate_a >> i) & 1u) && vf_frame(va[i], fr, lim)) hit_a |= 1ull << (8 * i + j);
     }
@@ -444,7 +444,7 @@ __device__ inline void for_each_feature(const PolyNbhArgs& a, int64_t x, uint32_
   if (gate_b) {
     const double lim = rb + ra + rv;
     for (int i = 0; i < sa.nf; i++) {
-      const FaceFrame fr = face_frame(va, sa, i);
+      const FaceFrame fr = face_frame(va, sa.faces[i], sa.face_size[i]);
       for (int j = 0; j < sb.nv; j++)
         if (((gate_b >> j) & 1u) && vf_frame(vb[j], fr, lim)) hit_b |= 1ull << (8 * j + i);
     }
@@ -511,45 +511,227 @@ __global__ __launch_bounds__(256) void k_owner_slots(NbrList nl, uint32_t* __res
   }
 }
 
-// One thread per owner slot: the pair's features enumerated once, the count and up to kFeatPerSlot
-// feature words kept in the slot's region of tmp.
+// Owner pairs whose enlarged boxes meet (the OBB test of for_each_feature), compacted again: one thread per owner slot,
+// one atomic per block. The others have no features (their counts stay zero).
+__global__ __launch_bounds__(256) void k_pair_gate(PolyNbhArgs a, const uint32_t* __restrict__ oslot,
+                                                   uint32_t* __restrict__ nown, uint32_t* __restrict__ gslot) {
+  __shared__ uint32_t wtot[4], bbase;
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t total = (int64_t)nown[0];
+  if ((int64_t)blockIdx.x * blockDim.x >= total) return;
+  bool meet = false;
+  uint32_t sl = 0;
+  if (t < total) {
+    sl = oslot[t];
+    const uint32_t x = a.nl.sx[sl], wd = a.nl.word[sl], y = wd & kIdxMask;
+    const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
+    const d4 xa = a.s.core[x].xr, xb = a.s.core[y].xr, qa = a.s.core[x].q, qb = a.s.core[y].q;
+    const double ha = a.s.core[x].w.w, hb = a.s.core[y].w.w;
+    OBBd oi = compute_obb(a.shapes[a.s.type[x]], V3{xa.x, xa.y, xa.z}, qa, ha);
+    OBBd oj = compute_obb(a.shapes[a.s.type[y]], V3{xb.x, xb.y, xb.z} + sh, qb, hb);
+    obb_enlarge(oi, 0.5 * a.rv);
+    obb_enlarge(oj, 0.5 * a.rv);
+    meet = obb_intersect(oi, oj);
+  }
+  const unsigned long long bal = __ballot(meet);
+  if (lane == 0) wtot[wv] = (uint32_t)__popcll(bal);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t tot = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+    bbase = tot ? atomicAdd(nown + 3, tot) : 0u;
+  }
+  __syncthreads();
+  uint32_t pos = bbase;
+  for (int w = 0; w < wv; w++) pos += wtot[w];
+  if (meet) gslot[pos + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = sl;
+}
+
+// The features of each pair, sixteen lanes per pair (four pairs per wavefront): lanes 0-7 take one vertex of the owner
+// each (box gate, VV, VE, VF against the partner), lanes 8-15 one vertex of the partner (the swap pass), lanes 0-11 one
+// edge of the owner (EE), and each lane the frame of one face of the other body; vertices, frames and the shapes' index
+// tables are shared through LDS. A lane's hits are bit masks; prefix sums over the pair's lanes put the words into the
+// order of for_each_feature. The count and up to kFeatPerSlot feature words go to the slot's region of tmp.
+// FP64 arithmetic bounds it (144 edge pairs, up to 96 vertex-edge and 14 face tests per cube pair). A lattice of spacing
+// 1.35 to 1.4: 163 us at 20k polyhedra, 1.37 ms at 200k (175 us and 1.49 ms with filter_ee on every edge pair); one
+// thread per pair (164 registers, three wavefronts per SIMD, one long chain per thread) took 360 us and 1.88 ms.
 constexpr int kFeatPerSlot = 24;
-// Features past kFeatPerSlot go to a chunk of kPoolChunk words claimed from a shared pool (counter
-// nown[2], capacity pool_cap) at the first one; fpool[sl] = the chunk, or ~0u when the pool is exhausted
-// or the pair has more than kFeatPerSlot + kPoolChunk features (then k_feat_overflow enumerates it again).
+// Features past kFeatPerSlot go to a chunk of kPoolChunk words claimed from a shared pool (counter nown[2], capacity
+// pool_cap); fpool[sl] = the chunk, or ~0u when the pool is exhausted or the pair has more than kFeatPerSlot + kPoolChunk
+// features (then k_feat_overflow enumerates it again).
 constexpr int kEnumBlock = 128;
+constexpr int kPairLanes = 16, kEnumPairs = kEnumBlock / kPairLanes;
 constexpr uint32_t kPoolChunk = 232;
-__global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, const uint32_t* __restrict__ oslot,
+constexpr int64_t kEnumBlocks = 256 * 8;  // resident blocks walk the pairs
+static_assert(XDEM_MAX_SHAPE_VERTICES <= 8 && XDEM_MAX_SHAPE_FACES <= 8 && XDEM_MAX_SHAPE_EDGES <= kPairLanes,
+              "one lane per vertex, face and edge");
+struct V3s {  // vertices in LDS
+  const V3* p;
+  __device__ V3 operator[](int k) const { return p[k]; }
+};
+// The shapes' index tables as bytes
+struct ShapeIdx {
+  uint8_t nv, ne, nf, pad;
+  uint8_t edge[XDEM_MAX_SHAPE_EDGES][2];
+  uint8_t fsize[XDEM_MAX_SHAPE_FACES];
+  uint8_t face[XDEM_MAX_SHAPE_FACES][XDEM_MAX_FACE_VERTICES];
+};
+// orders the LDS accesses of a pair's lanes, which lie in one wavefront (nothing is executed)
+__device__ inline void pair_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// inclusive prefix sum over the 16 lanes of a pair
+__device__ inline uint32_t pair_scan(uint32_t v, int l) {
+#pragma unroll
+  for (int o = 1; o < kPairLanes; o <<= 1) {
+    const uint32_t t = __shfl_up(v, o, kPairLanes);
+    if (l >= o) v += t;
+  }
+  return v;
+}
+__global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nshapes, const uint32_t* __restrict__ gslot,
                                                           uint32_t* __restrict__ nown, uint32_t* __restrict__ fcount,
                                                           uint32_t* __restrict__ tmp, uint32_t* __restrict__ pool,
                                                           uint32_t pool_cap, uint32_t* __restrict__ fpool) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)nown[0]) return;
-  const uint32_t sl = oslot[t];
-  const uint32_t x = a.nl.sx[sl], wd = a.nl.word[sl];
-  uint32_t nf = 0, pb = ~0u;
-  uint32_t* out = tmp + (int64_t)sl * kFeatPerSlot;
-  for_each_feature(a, x, wd & kIdxMask, (int)((wd >> kShiftShift) & 31u), [&](int ty, int sw, int si, int sj) {
-    const uint32_t w = sw ? feat_word(ty, 1, si, sj) : feat_word(ty, 0, si, sj);
-    if (nf < (uint32_t)kFeatPerSlot) {
-      out[nf] = w;
-    } else {
-      if (nf == (uint32_t)kFeatPerSlot) {
-        const uint32_t b = atomicAdd(nown + 2, kPoolChunk);
-        pb = b <= pool_cap - kPoolChunk ? b : ~0u;
-      }
-      if (pb != ~0u && nf < (uint32_t)kFeatPerSlot + kPoolChunk) pool[pb + (nf - kFeatPerSlot)] = w;
+  __shared__ ShapeIdx tab[XDEM_MAX_SHAPES];
+  __shared__ V3 verts[kEnumPairs][2][XDEM_MAX_SHAPE_VERTICES];
+  __shared__ FaceFrame frames[kEnumPairs][kPairLanes];
+  // sixteen lanes per shape: edge l and, in lanes 0-7, face l (unused entries stay unread)
+  for (int k = (int)threadIdx.x / kPairLanes; k < nshapes; k += kEnumPairs) {
+    const xdem_shape& sh = a.shapes[k];
+    ShapeIdx& t = tab[k];
+    const int q = (int)threadIdx.x & (kPairLanes - 1);
+    if (q == 0) {
+      t.nv = (uint8_t)sh.nv;
+      t.ne = (uint8_t)sh.ne;
+      t.nf = (uint8_t)sh.nf;
     }
-    nf++;
-  });
-  fcount[sl] = nf;
-  if (nf > (uint32_t)kFeatPerSlot) fpool[sl] = nf <= (uint32_t)kFeatPerSlot + kPoolChunk ? pb : ~0u;
+    if (q < XDEM_MAX_SHAPE_EDGES) {
+      t.edge[q][0] = (uint8_t)sh.edges[q][0];
+      t.edge[q][1] = (uint8_t)sh.edges[q][1];
+    }
+    if (q < XDEM_MAX_SHAPE_FACES) {
+      t.fsize[q] = (uint8_t)sh.face_size[q];
+#pragma unroll
+      for (int v = 0; v < XDEM_MAX_FACE_VERTICES; v++) t.face[q][v] = (uint8_t)sh.faces[q][v];
+    }
+  }
+  __syncthreads();
+  const int l = (int)threadIdx.x & (kPairLanes - 1), pr = (int)threadIdx.x / kPairLanes;
+  const bool own = l < 8;  // the lane's vertex is the owner's
+  const int vi = l & 7;
+  const double rv = a.rv;
+  const int64_t total = (int64_t)nown[3];
+  for (int64_t t = (int64_t)blockIdx.x * kEnumPairs + pr; t < total; t += (int64_t)gridDim.x * kEnumPairs) {
+    const uint32_t sl = gslot[t];
+    const uint32_t x = a.nl.sx[sl], wd = a.nl.word[sl], y = wd & kIdxMask;
+    const V3 sh = shift_vec(a.g, (int)((wd >> kShiftShift) & 31u));
+    const uint32_t ta = a.s.type[x], tb = a.s.type[y];
+    const xdem_shape &sa = a.shapes[ta], &sb = a.shapes[tb];
+    const ShapeIdx &ia = tab[ta], &ib = tab[tb];
+    const double ha = a.s.core[x].w.w, hb = a.s.core[y].w.w;
+    const double ra = sa.minkowski * ha, rb = sb.minkowski * hb;
+    // the lane's vertex, and the other body's box for its gate
+    const uint32_t mine = own ? x : y, other = own ? y : x;
+    const ShapeIdx &im = own ? ia : ib, &io = own ? ib : ia;
+    const bool has = vi < (int)im.nv;
+    const d4 v4 = a.vtx[(int64_t)mine * XDEM_MAX_SHAPE_VERTICES + (has ? vi : 0)];
+    const V3 v = own ? V3{v4.x, v4.y, v4.z} : V3{v4.x + sh.x, v4.y + sh.y, v4.z + sh.z};
+    const d4 xo = a.s.core[other].xr, qo = a.s.core[other].q;
+    const V3 po = own ? V3{xo.x, xo.y, xo.z} + sh : V3{xo.x, xo.y, xo.z};
+    OBBd box = compute_obb(own ? sb : sa, po, qo, own ? hb : ha);
+    obb_enlarge(box, 0.5 * rv);
+    obb_enlarge(box, 0.5 * rv);
+    pair_fence();
+    verts[pr][own ? 0 : 1][vi] = v;
+    pair_fence();
+    bool gate = false;
+    if (has) {
+      OBBd ov;
+      ov.c = v;
+      ov.e1 = {1, 0, 0};
+      ov.e2 = {0, 1, 0};
+      ov.e3 = {0, 0, 1};
+      ov.ext = {0, 0, 0};
+      obb_enlarge(ov, own ? ra : rb);
+      gate = obb_intersect(box, ov);
+    }
+    const V3s va{verts[pr][0]}, vb{verts[pr][1]};
+    const V3s vo = own ? vb : va;
+    // frames of the other body's faces, for the pair's lanes of this side (none without a gated vertex)
+    const uint64_t gates = __ballot(gate);
+    const uint32_t side = (uint32_t)(gates >> (((int)threadIdx.x & 63) & ~7)) & 0xffu;
+    if (side && vi < (int)io.nf) frames[pr][l] = face_frame(vo, io.face[vi], (int)io.fsize[vi]);
+    pair_fence();
+    uint32_t vv = 0, ve = 0, vf = 0, ee = 0;
+    if (gate) {
+      const double rs = own ? ra : rb, ro = own ? rb : ra;
+      if (own)
+        for (int j = 0; j < (int)ib.nv; j++)
+          if (filter_vv(rv, v, ra, vb[j], rb)) vv |= 1u << j;
+      for (int j = 0; j < (int)io.ne; j++)
+        if (filter_ve(rv, v, rs, vo[io.edge[j][0]], vo[io.edge[j][1]], ro)) ve |= 1u << j;
+      const double lim = rs + ro + rv;
+      for (int j = 0; j < (int)io.nf; j++)
+        if (vf_frame(v, frames[pr][(l & 8) + j], lim)) vf |= 1u << j;
+    }
+    if (l < (int)ia.ne) {
+      const V3 e0 = va[ia.edge[l][0]], e1 = va[ia.edge[l][1]];
+      // filter_ee's closest points lie on the two edges: edges whose boxes are further apart than its limit (and the
+      // rounding of the points, far below 1e-9 of the coordinates) cannot pass
+      const double lim = ra + rb + rv;
+      const double m = lim + 1e-9 * (lim + fabs(e0.x) + fabs(e0.y) + fabs(e0.z) + fabs(e1.x) + fabs(e1.y) + fabs(e1.z));
+      const V3 lo{fmin(e0.x, e1.x) - m, fmin(e0.y, e1.y) - m, fmin(e0.z, e1.z) - m};
+      const V3 hi{fmax(e0.x, e1.x) + m, fmax(e0.y, e1.y) + m, fmax(e0.z, e1.z) + m};
+      uint32_t near = 0;
+      for (int j = 0; j < (int)ib.ne; j++) {
+        const V3 p = vb[ib.edge[j][0]], q = vb[ib.edge[j][1]];
+        const bool far = fmax(p.x, q.x) < lo.x || fmin(p.x, q.x) > hi.x || fmax(p.y, q.y) < lo.y ||
+                         fmin(p.y, q.y) > hi.y || fmax(p.z, q.z) < lo.z || fmin(p.z, q.z) > hi.z;
+        if (!far) near |= 1u << j;
+      }
+      for (; near; near &= near - 1u) {
+        const int j = __ffs(near) - 1;
+        if (filter_ee(rv, e0, e1, ra, vb[ib.edge[j][0]], vb[ib.edge[j][1]], rb)) ee |= 1u << j;
+      }
+    }
+    // positions: the owner's vertices, the edges, the partner's vertices
+    const uint32_t nv_ = (uint32_t)(__popc(vv) + __popc(ve) + __popc(vf)), ne_ = (uint32_t)__popc(ee);
+    const uint32_t sv = pair_scan(nv_, l), se = pair_scan(ne_, l);
+    const uint32_t tv = __shfl(sv, 7, kPairLanes), te = __shfl(se, kPairLanes - 1, kPairLanes);
+    const uint32_t nf = __shfl(sv, kPairLanes - 1, kPairLanes) + te;
+    uint32_t pb = ~0u;
+    if (l == 0) {
+      fcount[sl] = nf;
+      if (nf > (uint32_t)kFeatPerSlot) {
+        if (nf <= (uint32_t)kFeatPerSlot + kPoolChunk) {
+          const uint32_t b = atomicAdd(nown + 2, kPoolChunk);
+          pb = b <= pool_cap - kPoolChunk ? b : ~0u;
+        }
+        fpool[sl] = pb;
+      }
+    }
+    pb = __shfl(pb, 0, kPairLanes);
+    uint32_t* out = tmp + (int64_t)sl * kFeatPerSlot;
+    uint32_t at = sv - nv_ + (own ? 0u : te);
+    auto put = [&](uint32_t w) {
+      if (at < (uint32_t)kFeatPerSlot) out[at] = w;
+      else if (pb != ~0u) pool[pb + (at - kFeatPerSlot)] = w;
+      at++;
+    };
+    for (; vv; vv &= vv - 1u) put(feat_word(0, 0, vi, __ffs(vv) - 1));
+    for (; ve; ve &= ve - 1u) put(own ? feat_word(1, 0, vi, __ffs(ve) - 1) : feat_word(1, 1, __ffs(ve) - 1, vi));
+    for (; vf; vf &= vf - 1u) put(own ? feat_word(2, 0, vi, __ffs(vf) - 1) : feat_word(2, 1, __ffs(vf) - 1, vi));
+    at = tv + se - ne_;
+    for (; ee; ee &= ee - 1u) put(feat_word(3, 0, l, __ffs(ee) - 1));
+  }
 }
 
-// One thread per owner slot: its feature words copied to their place in the list (slot order, from the
+// One thread per pair of k_feat_enum: its feature words copied to their place in the list (slot order, from the
 // scan of the counts), the first kFeatPerSlot from tmp and the rest from its pool chunk; a pair without a
 // chunk goes to the overflow list (count in nown[1]) for k_feat_overflow.
-__global__ __launch_bounds__(256) void k_feat_place(NbrList nl, const uint32_t* __restrict__ oslot,
+__global__ __launch_bounds__(256) void k_feat_place(NbrList nl, const uint32_t* __restrict__ gslot,
                                                     uint32_t* __restrict__ nown, const uint32_t* __restrict__ fcount,
                                                     const uint32_t* __restrict__ tmp, const uint32_t* __restrict__ pool,
                                                     const uint32_t* __restrict__ fpool,
@@ -557,8 +739,8 @@ __global__ __launch_bounds__(256) void k_feat_place(NbrList nl, const uint32_t* 
                                                     uint32_t* __restrict__ fslot, uint32_t* __restrict__ fown,
                                                     uint32_t* __restrict__ ovf) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)nown[0]) return;
-  const uint32_t sl = oslot[t];
+  if (t >= (int64_t)nown[3]) return;
+  const uint32_t sl = gslot[t];
   const uint32_t nf = fcount[sl];
   if (nf == 0) return;
   const uint32_t pb = nf > (uint32_t)kFeatPerSlot ? fpool[sl] : 0u;
@@ -1014,7 +1196,7 @@ int poly_nbh(xdem_ctx* c, double rcut_inc) {
     int64_t pcap = std::min<int64_t>(cap / 128 * kPoolChunk + 64 * kPoolChunk, 0x7fffffffLL);
     if (const char* e = std::getenv("XDEM_FEAT_POOL_WORDS"))
       pcap = std::min<int64_t>(std::max<int64_t>(std::atoll(e), kPoolChunk), 0x7fffffffLL);
-    if ((rc = galloc(c, &c->oslot, cap)) || (rc = galloc(c, &c->feat_ovf, cap)) ||
+    if ((rc = galloc(c, &c->oslot, cap)) || (rc = galloc(c, &c->gslot, cap)) || (rc = galloc(c, &c->feat_ovf, cap)) ||
         (rc = galloc(c, &c->feat_fpool, cap)) || (rc = galloc(c, &c->feat_pool, pcap)))
       return rc;
     c->cap_oslot = cap;
@@ -1028,9 +1210,11 @@ int poly_nbh(xdem_ctx* c, double rcut_inc) {
   if (n > 0) {
     hipLaunchKernelGGL(k_owner_slots, dim3(grid_blocks(std::max<int64_t>(L.slots, 1), 256 * kOwnChunk)), dim3(256), 0,
                        c->stream, L, c->oslot, c->d_nown);
-    hipLaunchKernelGGL(k_feat_enum, dim3(grid_blocks(std::max<int64_t>(L.slots, 1), kEnumBlock)), dim3(kEnumBlock), 0,
-                       c->stream, a, c->oslot, c->d_nown, P.fcount, c->feat_tmp, c->feat_pool,
-                       (uint32_t)c->cap_feat_pool, c->feat_fpool);
+    // about half of the slots are owner slots (both, for periodic images); blocks past their number return at once
+    hipLaunchKernelGGL(k_pair_gate, gsl, bsl, 0, c->stream, a, c->oslot, c->d_nown, c->gslot);
+    const int64_t eblk = std::min<int64_t>(grid_blocks(std::max<int64_t>(L.slots, 1), kEnumPairs), kEnumBlocks);
+    hipLaunchKernelGGL(k_feat_enum, dim3((uint32_t)eblk), dim3(kEnumBlock), 0, c->stream, a, c->nshapes, c->gslot,
+                       c->d_nown, P.fcount, c->feat_tmp, c->feat_pool, (uint32_t)c->cap_feat_pool, c->feat_fpool);
     if ((rc = scan_u64_from_u32(c, P.fcount, P.start, L.slots, 1u))) return rc;
   }
   uint64_t nf = 0;
@@ -1053,7 +1237,7 @@ int poly_nbh(xdem_ctx* c, double rcut_inc) {
   if (nf >= 0xffffffffull) return set_err(c, XDEM_ERR_CAPACITY, "nbh_polyhedron: more than 2^32 - 2 features");
   P.nfeat = (int64_t)nf;
   if (n > 0) {
-    hipLaunchKernelGGL(k_feat_place, gsl, bsl, 0, c->stream, L, c->oslot, c->d_nown, P.fcount, c->feat_tmp,
+    hipLaunchKernelGGL(k_feat_place, gsl, bsl, 0, c->stream, L, c->gslot, c->d_nown, P.fcount, c->feat_tmp,
                        c->feat_pool, c->feat_fpool, P.start, P.feat, P.fslot, P.fown, c->feat_ovf);
     hipLaunchKernelGGL(k_feat_overflow, dim3(kOvfBlocks), dim3(kEnumBlock), 0, c->stream, a, c->d_nown, c->feat_ovf,
                        P.start, P.feat, P.fslot, P.fown);

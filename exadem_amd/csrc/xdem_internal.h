@@ -471,12 +471,13 @@ struct xdem_ctx {
   uint32_t* feat_tmp = nullptr;     // [cap_feat_tmp] per list slot, up to kFeatPerSlot feature words of the
   int64_t cap_feat_tmp = 0;         // one-pass enumeration (nbh_polyhedron)
   uint32_t* oslot = nullptr;        // [cap_oslot] owner slots of the list (nbh_polyhedron)
+  uint32_t* gslot = nullptr;        // [cap_oslot] those of them whose pair's boxes meet
   uint32_t* feat_ovf = nullptr;     // [cap_oslot] owner slots whose features are enumerated again
   uint32_t* feat_fpool = nullptr;   // [cap_oslot] per slot: its chunk of feat_pool (features past the tmp region)
   uint32_t* feat_pool = nullptr;    // [cap_feat_pool]
   int64_t cap_feat_pool = 0;
   int64_t cap_oslot = 0;
-  uint32_t* d_nown = nullptr;       // their number
+  uint32_t* d_nown = nullptr;       // [4] owner slots, overflowing pairs, pool words claimed, pairs whose boxes meet
   uint2* frange = nullptr;          // [cap_frange] per list slot: first feature and count of its pair
                                     // (through the owner entry for partner entries); x = ~0u: no owner entry
   int64_t cap_frange = 0;

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from exadem_amd import inputs, native
+from exadem_amd import shapes as shp
 from exadem_amd.sim import PolySim, scheme
 import pyoracle as po
 
@@ -370,3 +371,28 @@ def test_integrating_gather_matches_oracle(gpu_ok, n):
     gk, gf = feature_table(*s.ctx.poly_interactions())
     ok, of = feature_table(*o.poly_interactions())
     assert np.array_equal(gk, ok) and np.array_equal(gf, of) and np.count_nonzero(gf) > 0
+
+
+@pytest.mark.parametrize("n", [2, 9, 77, 1203])
+def test_feature_enumeration_of_mixed_shapes(gpu_ok, n):
+    """Sixteen lanes per pair: shapes that fill all vertex, edge and face lanes (cube, octahedron) and shapes that leave
+    most of them idle (a rod: two vertices, one edge, no face; a sphere: one vertex), with numbers of pairs below and
+    beyond a block: the feature lists equal the oracle's, word for word and in order."""
+    rod, ball = shp.ShapeDef("rod"), shp.ShapeDef("sphere")
+    rod.vertices, rod.edges = [(-0.6, 0.0, 0.0), (0.6, 0.0, 0.0)], [(0, 1)]
+    ball.vertices = [(0.0, 0.0, 0.0)]
+    for d, r in ((rod, 0.05), (ball, 0.4)):
+        d.radius, d.volume, d.inertia_on_mass = r, 0.2, (0.1, 0.1, 0.1)
+    w = inputs.polyhedra(density=2500.0, n=n, spacing=1.1, jitter=0.05, seed=n, dt=2e-4, z0=0.8,
+                         periodic=(n > 500, n > 500, False))
+    w.shapes = list(w.shapes) + [rod.to_record(), ball.to_record()]
+    w.particles["type"] = (np.arange(n) * 7 // 3 % 4).astype(np.uint32)
+    o = oracle_for(w)
+    o.rebuild_poly(w.rcut_inc)
+    s = PolySim(w)
+    s.rebuild()
+    gk, gf = feature_table(*s.ctx.poly_interactions())
+    ok, of = feature_table(*o.poly_interactions())
+    assert np.array_equal(gk, ok) and np.array_equal(gf, of)
+    if n > 500:
+        assert {0, 1, 2, 3} <= set(gk[:, 2]) and set(gk[gk[:, 2] > 0, 3]) == {0, 1}
