@@ -354,30 +354,29 @@ __global__ __launch_bounds__(256) void k_nbh_rows(CellNbhArgs a) {
 // 128 / 256 / 512 / 1024 / 2048.
 constexpr int kBalance = 256;
 constexpr int kBalanceBins = 64;
-__global__ __launch_bounds__(64) void k_balance(int64_t n, const uint32_t* __restrict__ cnt,
-                                                uint32_t* __restrict__ perm2, uint32_t* __restrict__ inv2) {
-  __shared__ uint32_t start[kBalanceBins];
-  __shared__ uint8_t bin[kBalance];
+// One thread per particle: its place is the number of smaller keys (bin, then Morton order) in the group, counted over
+// the keys in LDS. (One thread sorting its group serially took 24 us whatever the particle number.)
+__global__ __launch_bounds__(kBalance) void k_balance(int64_t n, const uint32_t* __restrict__ cnt,
+                                                      uint32_t* __restrict__ perm2, uint32_t* __restrict__ inv2) {
+  __shared__ uint4 keys[kBalance / 4];
   const int64_t g0 = (int64_t)blockIdx.x * kBalance;
-  const int m = (int)(((g0 + kBalance) < n ? (g0 + kBalance) : n) - g0);
-  for (int i = threadIdx.x; i < m; i += 64) {
-    const uint32_t c = cnt[g0 + i];
-    bin[i] = (uint8_t)(kBalanceBins - 1 - (c < kBalanceBins ? c : kBalanceBins - 1));  // longest lists first
+  const int64_t i = g0 + threadIdx.x;
+  uint32_t key = ~0u;  // past the end: after every particle
+  if (i < n) {
+    const uint32_t c = cnt[i];
+    key = (kBalanceBins - 1 - (c < kBalanceBins ? c : kBalanceBins - 1)) * kBalance + threadIdx.x;  // longest first
   }
+  ((uint32_t*)keys)[threadIdx.x] = key;
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int b = 0; b < kBalanceBins; b++) start[b] = 0;
-  for (int i = 0; i < m; i++) start[bin[i]]++;
-  uint32_t run = (uint32_t)g0;
-  for (int b = 0; b < kBalanceBins; b++) {
-    const uint32_t t = start[b];
-    start[b] = run;
-    run += t;
+  uint32_t rank = 0;
+#pragma unroll 8
+  for (int k = 0; k < kBalance / 4; k++) {
+    const uint4 q = keys[k];
+    rank += (q.x < key) + (q.y < key) + (q.z < key) + (q.w < key);
   }
-  for (int i = 0; i < m; i++) {
-    const uint32_t pos = start[bin[i]]++;
-    perm2[pos] = (uint32_t)(g0 + i);
-    inv2[g0 + i] = pos;
+  if (i < n) {
+    perm2[g0 + rank] = (uint32_t)i;
+    inv2[i] = (uint32_t)(g0 + rank);
   }
 }
 
@@ -545,7 +544,7 @@ int do_chunk_neighbors(xdem_ctx* c, double rcut_inc, double nbh_dist) {
   const int64_t nseg = (int64_t)((g.dims[0] + kRowCells - 1) / kRowCells) * g.dims[1] * g.dims[2];
   const dim3 cgrid((uint32_t)((nseg + 3) / 4));
   hipLaunchKernelGGL(k_nbh_rows, cgrid, dim3(256), 0, c->stream, a);
-  hipLaunchKernelGGL(k_balance, dim3(grid_blocks(n, kBalance)), dim3(64), 0, c->stream, n, cnt_m, perm2, inv2);
+  hipLaunchKernelGGL(k_balance, dim3(grid_blocks(n, kBalance)), dim3(kBalance), 0, c->stream, n, cnt_m, perm2, inv2);
   hipLaunchKernelGGL(k_balance_apply, dim3(grid_blocks(n, 256)), dim3(256), 0, c->stream, n, perm2, cnt_m, L.cnt,
                      L.kmax, c->perm, perm_tmp);
   hipLaunchKernelGGL(k_max_u32, dim3(1), dim3(1024), 0, c->stream, nw, L.kmax, max_rows);
