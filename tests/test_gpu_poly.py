@@ -396,3 +396,21 @@ def test_feature_enumeration_of_mixed_shapes(gpu_ok, n):
     assert np.array_equal(gk, ok) and np.array_equal(gf, of)
     if n > 500:
         assert {0, 1, 2, 3} <= set(gk[:, 2]) and set(gk[gk[:, 2] > 0, 3]) == {0, 1}
+
+
+@pytest.mark.parametrize("n", [41, 1203])
+def test_histories_carried_over_rebuilds(gpu_ok, n):
+    """Histories found again by feature: after several rebuilds with pairs in contact the lists and friction histories
+    equal the oracle's bit for bit, over more or fewer features than a block."""
+    w = inputs.polyhedra(density=2500.0, n=n, spacing=1.3, jitter=0.05, seed=n, dt=5e-4, sigma_v=3.0, z0=0.7,
+                         periodic=(n > 500, n > 500, False))
+    s = PolySim(w)
+    s.first_iteration()
+    st = s.run(60, poll=16)
+    o = oracle_for(w)
+    o.first_iteration_poly(scheme(w))
+    o.run_steps_poly(scheme(w), 60)
+    gk, gf = feature_table(*s.ctx.poly_interactions())
+    ok, of = feature_table(*o.poly_interactions())
+    assert st["rebuilds"] >= 2
+    assert np.array_equal(gk, ok) and np.array_equal(gf, of) and np.count_nonzero(gf) > 0
