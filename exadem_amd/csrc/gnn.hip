@@ -544,6 +544,21 @@ __device__ inline void ld2(const uint16_t* p, float& a, float& b) {
   b = bf2f((uint16_t)(v >> 16));
 }
 
+// orders this wavefront's LDS accesses across its lanes (nothing is executed)
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// max(x, 0), NaN -> 0, in one instruction (fmaxf on a matrix instruction's result costs a second one that quiets its
+// operand). inf: an infinity that the compiler does not see, or it writes the median back as that maximum.
+__device__ inline float hidden_inf() {
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return inf;
+}
+__device__ inline float relu(float x, float inf) { return __builtin_amdgcn_fmed3f(x, 0.f, inf); }
+
 // Message pass on MFMA: one block of four wavefronts per 32 consecutive particles (half of a
 // 64-particle list group), each wavefront for 32 of the 128 channels. Step k takes neighbour rank k
 // of each of the 32 particles, i.e. 32 consecutive list slots, and computes D[row][edge] =
@@ -553,39 +568,25 @@ __device__ inline void ld2(const uint16_t* p, float& a, float& b) {
 // added on the matrix unit; relu(z) is summed over k in the accumulator layout. Accumulator element
 // v of lane l is row 8*(v/4) + 4*(l/32) + v%4 of edge column l%32; rows are mapped to channels by
 // c(8g + 4h + q) = 16h + 4g + q inside the 32-channel tile, so that lane half h holds the 16
-// consecutive channels 16h..16h+15 (16-byte loads of P, 16-byte stores of m). The list words and edge inputs of the block's 32 slots are shared by its four
-// wavefronts through L1. The list word, edge inputs and Q rows of step k+1 are requested before
-// step k is computed, the list word of step k+2 before that.
-struct MsgStep {
-  bool ok;
-  bf16x8 eb;
-  uint4 q[2];
-};
-__device__ inline void msg_load(const MsgArgs& a, uint64_t sl, bool ok, uint32_t wd, int half, int ch0, uint32_t self,
-                                MsgStep& st) {
-  st.ok = ok;
-  (void)self;
-  if (ok) {
-    st.eb = *(const bf16x8*)(a.e + sl * FE + 8 * half);
-    const uint16_t* qrow = a.pq + (int64_t)(wd & kIdxMask) * H2 + H + ch0 + 8 * half;
-    st.q[0] = *(const uint4*)(qrow);
-    st.q[1] = *(const uint4*)(qrow + 16);
-  } else {
-    // padding slot of the list group: nothing is gathered (its column of the MFMA is not summed)
-#pragma unroll
-    for (int q = 0; q < 8; q++) st.eb[q] = (__bf16)0.0f;
-    st.q[0] = uint4{0u, 0u, 0u, 0u};
-    st.q[1] = uint4{0u, 0u, 0u, 0u};
-  }
-}
+// consecutive channels 16h..16h+15 (16-byte loads of P, 16-byte stores of m). Edge inputs and Q rows
+// of step k+1 are requested before step k is computed, the list words of step k+2 before that.
+//
+// The Q rows bound it: a wavefront's 64 bytes of a row are loaded by four neighbouring lanes and pass through
+// its own LDS rows into the MFMA layout (chunk c of row r at c ^ (r/4 % 4): neither the stores nor the loads meet a
+// bank twice), which takes a quarter of the cache accesses that 16-byte loads straight into the layout (one edge
+// per lane) took: 74M -> 42M accesses of all kinds at 500k spheres, 239 -> 208 us per layer, and 86 -> 72 us at 200k.
+// Launch bounds of four blocks keep the accumulators in VGPRs (the accumulation registers cost a move per value).
+// Requesting two steps ahead, or five blocks per CU, gained nothing; loading the padding slots too, so that no load
+// stands behind a branch, cost more (247 us) than the deeper queue gave.
 __device__ inline float bf_lo(uint32_t v) { return bf2f((uint16_t)(v & 0xffffu)); }
 __device__ inline float bf_hi(uint32_t v) { return bf2f((uint16_t)(v >> 16)); }
 
-__global__ __launch_bounds__(256) void k_msg_fwd_mfma(MsgArgs a, const uint16_t* __restrict__ wEb) {
-  const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(256, 4) void k_msg_fwd_mfma(MsgArgs a, const uint16_t* __restrict__ wEb) {
+  __shared__ uint4 qs[4][2][kWave];  // per wavefront: 32 rows x 4 chunks of 8 channels
+  const int lane = threadIdx.x & 63, wv = (int)(threadIdx.x >> 6);
   // XCD-aware block order: consecutive particle groups on one XCD share its L2 for the Q gathers
   const int64_t i0 = xcd_block(blockIdx.x, gridDim.x) * 32;
-  const int ch0 = (int)(threadIdx.x >> 6) * 32;
+  const int ch0 = wv * 32;
   if (i0 >= a.n) return;
   const int col = lane & 31, half = lane >> 5;
   const int64_t i = i0 + col;
@@ -595,6 +596,16 @@ __global__ __launch_bounds__(256) void k_msg_fwd_mfma(MsgArgs a, const uint16_t*
   const uint64_t base = a.nl.base[grp] + (uint64_t)(ic & 63);
   const uint32_t cnt = vi ? a.nl.cnt[ic] : 0u;
   const uint32_t kmax = a.nl.kmax[grp];
+  // the two list rows whose Q chunk this lane loads: rows lane/4 and 16 + lane/4 of the block's 32
+  const int64_t r0 = i0 + (lane >> 2), r1 = r0 + 16;
+  const uint32_t cnt0 = r0 < a.n ? a.nl.cnt[r0] : 0u, cnt1 = r1 < a.n ? a.nl.cnt[r1] : 0u;
+  const uint32_t* w0 = a.nl.word + a.nl.base[grp] + (uint64_t)(r0 & 63);
+  const uint32_t* w1 = w0 + 16;
+  // which chunk it takes, and where the chunks of its own column lie: chunk c of row r is at c ^ (r / 4 % 4)
+  const uint16_t* qbase = a.pq + H + ch0 + 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  const int sw = (col >> 2) & 3;
+  uint4* qw = &qs[wv][0][0];
+  const uint4 *qr0 = qw + 4 * col + (half ^ sw), *qr1 = qw + 4 * col + ((2 + half) ^ sw);
   // A rows: MFMA row `col` of the tile is channel c(col)
   const int crow = 16 * ((col >> 2) & 1) + 4 * (col >> 3) + (col & 3);
   const bf16x8 wa = *(const bf16x8*)(wEb + (ch0 + crow) * FE + 8 * half);
@@ -622,27 +633,36 @@ __global__ __launch_bounds__(256) void k_msg_fwd_mfma(MsgArgs a, const uint16_t*
 #pragma unroll
     for (int v = 0; v < 16; v++) msum[v] = 0.f;
   }
-  MsgStep cur, nxt;
-  uint32_t wnext = 0;
-  if (kmax > 0) {
-    const uint32_t w0 = cnt > 0 ? a.nl.word[base] : 0u;
-    msg_load(a, base, cnt > 0, w0, half, ch0, (uint32_t)ic, cur);
-    if (kmax > 1 && cnt > 1) wnext = a.nl.word[base + kWave];
-  }
+  const float inf = hidden_inf();
+  // a padding slot's chunk and edge inputs keep an earlier entry's (or zero) values: its column is not summed
+  uint4 q0{0u, 0u, 0u, 0u}, q1{0u, 0u, 0u, 0u}, en{0u, 0u, 0u, 0u};
+  uint32_t n0 = 0u, n1 = 0u;  // the list words of the step to load next
+  const uint16_t* ep = a.e + base * FE + 8 * half;
+  if (cnt0 > 0) n0 = w0[0];
+  if (cnt1 > 0) n1 = w1[0];
+  auto load = [&](uint32_t k) {
+    if (k < cnt0) q0 = *(const uint4*)(qbase + (int64_t)(n0 & kIdxMask) * H2);
+    if (k < cnt1) q1 = *(const uint4*)(qbase + (int64_t)(n1 & kIdxMask) * H2);
+    if (k < cnt) en = *(const uint4*)(ep + (uint64_t)k * (kWave * FE));
+    if (k + 1 < cnt0) n0 = w0[(uint64_t)(k + 1) * kWave];
+    if (k + 1 < cnt1) n1 = w1[(uint64_t)(k + 1) * kWave];
+  };
+  load(0);
   for (uint32_t k = 0; k < kmax; k++) {
-    if (k + 1 < kmax) {
-      const uint64_t sl1 = base + (uint64_t)(k + 1) * kWave;
-      msg_load(a, sl1, k + 1 < cnt, wnext, half, ch0, (uint32_t)ic, nxt);
-      wnext = (k + 2 < kmax && k + 2 < cnt) ? a.nl.word[sl1 + kWave] : 0u;
-    }
-    floatx16 d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa, cur.eb, cinit, 0, 0, 0);
-    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wia, __builtin_bit_cast(bf16x8, cur.q[0]), d, 0, 0, 0);
-    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wib, __builtin_bit_cast(bf16x8, cur.q[1]), d, 0, 0, 0);
-    if (cur.ok) {
+    qw[lane] = q0;
+    qw[kWave + lane] = q1;
+    const bf16x8 eb = __builtin_bit_cast(bf16x8, en);
+    load(k + 1);
+    wave_fence();
+    const bf16x8 x0 = __builtin_bit_cast(bf16x8, *qr0), x1 = __builtin_bit_cast(bf16x8, *qr1);
+    wave_fence();
+    floatx16 d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa, eb, cinit, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wia, x0, d, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wib, x1, d, 0, 0, 0);
+    if (k < cnt) {
 #pragma unroll
-      for (int v = 0; v < 16; v++) msum[v] += fmaxf(d[v], 0.f);
+      for (int v = 0; v < 16; v++) msum[v] += relu(d[v], inf);
     }
-    cur = nxt;
   }
   if (!vi) return;
   uint32_t o[8];
@@ -693,11 +713,6 @@ __device__ inline void bwd_load(const MsgArgs& a, uint64_t sl, bool ok, uint32_t
 __device__ int amdgcn_writelane(int val, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 __device__ inline uint32_t write_lane(uint32_t old, uint32_t val, int lane) {
   return (uint32_t)amdgcn_writelane((int)val, lane, (int)old);
-}
-// orders this wavefront's LDS accesses across its lanes (nothing is executed)
-__device__ inline void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
 }
 __device__ inline bf16x8 as_frag(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
 
