@@ -115,8 +115,11 @@ __device__ __forceinline__ void pair_fp64(const ForceArgs& a, uint64_t sl, const
     const double meff = (mi * mj) / (mi + mj);
     V3 ft = e.ft;
     V3 mint = e.mint;
-    const V3 f = owner ? hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vx, wx, rj, vy, wy)
-                       : hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vy, wy, rj, vx, wx);
+    // One call with the orientation selected: a wavefront holds owned and partner-owned entries, and a call per
+    // orientation ran the law twice (periodic packing, FP64: 28.4 -> 26.3 us per step at 120k spheres, 174 -> 169 at 1M;
+    // deposition unchanged within 1 %).
+    const V3 vi = owner ? vx : vy, wi = owner ? wx : wy, vj = owner ? vy : vx, wj = owner ? wy : wx;
+    const V3 f = hooke_force<KR>(dn, nrm, a.dt, a.cp, meff, ft, mint, cpos, ri, vi, wi, rj, vj, wj);
     if (REC && a.cstate && owner) {
       // the tuple the reference's functor returns for analyses: dn, contact point, f - ft, ft
       // (contact_sphere.hpp:175-202), with the two positions the interaction dump writes
