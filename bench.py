@@ -44,20 +44,17 @@ def bytes_model_poly(n, entries, nfeat, contacts, nvert=7.0):
     """Algorithmic HBM bytes per step of the polyhedra path (FP64), per kernel: what each kernel must move
     at least once.
 
-    k_poly_vertices, per particle: the record's position, spin/homothety and orientation (96 B), type (4 B),
-    the rebuild reference read (position 24 B + orientation 32 B), the world vertices written (32 B each,
-    nvert per particle on average: 8 for a cube, 6 for an octahedron).
-    k_poly_feat, per particle: its record (128 B) and vertices (32 B each) read once; per feature: the
-    classifier entry (16 B), the contact flag (1 B) and dn (8 B) written; per feature in contact: the
-    friction history read and written (48 B) and its force and moment terms written (72 B).
-    k_poly_gather, per particle: record (128 B), inertia (24 B), list length (4 B), the accelerations,
-    moments and angular accelerations written (72 B); per list entry: word and feature range (12 B); per
-    feature: the contact flag (1 B); per feature in contact: its terms read (72 B)."""
-    verts = (96 + 4 + 56 + 32 * nvert) * n
+    k_poly_feat, per particle: its record (128 B) and vertices (32 B each, nvert per particle on average: 8 for
+    a cube, 6 for an octahedron) read once; per feature: the classifier entry (16 B), the contact flag (1 B)
+    and dn (8 B) written; per feature in contact: the friction history read and written (48 B) and its force
+    and moment terms written (72 B).
+    k_poly_gather, which also integrates the particle, per particle: record read and written (256 B), inertia
+    (24 B), list length and type (8 B), the rebuild reference (position 24 B + orientation 32 B), the next
+    vertices written (32 B each); per list entry: word and feature range (12 B); per feature: the contact flag
+    (1 B); per feature in contact: its terms read (72 B)."""
     feat = (128 + 32 * nvert) * n + 25 * nfeat + 120 * contacts
-    gather = (128 + 24 + 4 + 72) * n + 12 * entries + nfeat + 72 * contacts
-    return {"k_poly_vertices": verts, "k_poly_feat": feat, "k_poly_gather": gather,
-            "force_pass": feat + gather, "step": verts + feat + gather}
+    gather = (256 + 24 + 8 + 56 + 32 * nvert) * n + 12 * entries + nfeat + 72 * contacts
+    return {"k_poly_feat": feat, "k_poly_gather": gather, "force_pass": feat + gather, "step": feat + gather}
 
 
 def profiled_traffic(stem):

@@ -4,7 +4,7 @@
 (data/config/main-config.msp:55-65 and data/config/config_numerical_schemes.msp:6-28, with
 compute_force = [gravity_force, contact_sphere] and the rebuild branch of
 config_move_particles.msp:141-195). `run` hands whole blocks of steps to the fused engine
-(xdem_run_steps), which produces the same state with two kernels per step.
+(xdem_run_steps), which produces the same state with one kernel per step.
 """
 import copy
 
