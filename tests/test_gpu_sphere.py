@@ -715,3 +715,28 @@ def test_step_lane_splits_match_oracle(gpu_ok, n):
     f.run(6, poll=3)
     c = by_id(f.ctx.download())
     assert rel_err(force(c), force(a), 9.81) <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 257, 3000])
+def test_partial_downloads_between_steps(gpu_ok, n):
+    """A download of the ids alone, of a few fields and of everything agree, and downloads between steps (whose staging
+    is the idle state's records, which the next rebuild rewrites) leave the run as it is without them."""
+    w = inputs.deposition(n=n, spacing=0.98, seed=n, start=0.48, box=(20.0, 20.0, 40.0))
+    w.particles["vx"] = np.full(n, 0.7 * w.rcut_inc / (40 * w.dt))  # past the rebuild threshold in every run below
+    a, b = gpu_for(w), gpu_for(w)
+    a.first_iteration()
+    b.first_iteration()
+    for _ in range(3):
+        for fields in (("id",), ("rx", "qw", "momx", "id")):
+            part = {k: np.zeros(n, np.uint64 if k == "id" else np.float64) for k in fields}
+            p, keep = native.particles_struct(part, n)
+            a.ctx.call("xdem_particles_download", native.C.byref(p))
+            full = a.ctx.download()
+            for k in fields:
+                assert np.array_equal(part[k], full[k]), k
+        a.run(40, poll=16)
+        b.run(40, poll=16)
+    assert a.rebuilds == b.rebuilds and a.rebuilds > 0
+    pa, pb = a.ctx.download(), b.ctx.download()
+    for k in pa:
+        assert np.array_equal(pa[k], pb[k]), k
