@@ -727,8 +727,12 @@ int xdem_particles_upload(xdem_ctx* c, const xdem_particles* p) {
     }
   }
   c->max_type = 0;
+  c->type_mask = p->type ? 0u : 1u;
   if (p->type)
-    for (int64_t i = 0; i < n; i++) c->max_type = std::max(c->max_type, p->type[i]);
+    for (int64_t i = 0; i < n; i++) {
+      c->max_type = std::max(c->max_type, p->type[i]);
+      c->type_mask |= 1u << std::min(p->type[i], 31u);
+    }
   XDEM_HIP(c, hipMemcpyAsync(s.type, p->type ? p->type : z32.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice,
                              c->stream));
   XDEM_HIP(c, hipMemcpyAsync(s.group, p->group ? p->group : z32.data(), sizeof(uint32_t) * n,

@@ -547,11 +547,12 @@ __global__ __launch_bounds__(256) void k_pair_gate(PolyNbhArgs a, const uint32_t
   if (meet) gslot[pos + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = sl;
 }
 
-// The features of each pair, sixteen lanes per pair (four pairs per wavefront): lanes 0-7 take one vertex of the owner
-// each (box gate, VV, VE, VF against the partner), lanes 8-15 one vertex of the partner (the swap pass), lanes 0-11 one
-// edge of the owner (EE), and each lane the frame of one face of the other body; vertices, frames and the shapes' index
-// tables are shared through LDS. A lane's hits are bit masks; prefix sums over the pair's lanes put the words into the
-// order of for_each_feature. The count and up to kFeatPerSlot feature words go to the slot's region of tmp.
+// The features of each pair, G lanes per pair (sixteen: four pairs per wavefront): the first half takes one vertex of the
+// owner each (box gate, VV, VE, VF against the partner), the second one vertex of the partner (the swap pass), the first
+// lanes of the pair one edge of the owner each (EE), and each lane the frame of one face of the other body; vertices,
+// frames and the shapes' index tables are shared through LDS. A lane's hits are bit masks; prefix sums over the pair's
+// lanes put the words into the order of for_each_feature. The count and up to kFeatPerSlot feature words go to the slot's
+// region of tmp.
 // FP64 arithmetic bounds it (144 edge pairs, up to 96 vertex-edge and 14 face tests per cube pair). A lattice of spacing
 // 1.35 to 1.4: 163 us at 20k polyhedra, 1.37 ms at 200k (175 us and 1.49 ms with filter_ee on every edge pair); one
 // thread per pair (164 registers, three wavefronts per SIMD, one long chain per thread) took 360 us and 1.88 ms.
@@ -560,7 +561,7 @@ constexpr int kFeatPerSlot = 24;
 // pool_cap); fpool[sl] = the chunk, or ~0u when the pool is exhausted or the pair has more than kFeatPerSlot + kPoolChunk
 // features (then k_feat_overflow enumerates it again).
 constexpr int kEnumBlock = 128;
-constexpr int kPairLanes = 16, kEnumPairs = kEnumBlock / kPairLanes;
+constexpr int kPairLanes = 16;  // the most lanes per pair
 constexpr uint32_t kPoolChunk = 232;
 constexpr int64_t kEnumBlocks = 256 * 8;  // resident blocks walk the pairs
 static_assert(XDEM_MAX_SHAPE_VERTICES <= 8 && XDEM_MAX_SHAPE_FACES <= 8 && XDEM_MAX_SHAPE_EDGES <= kPairLanes,
@@ -581,24 +582,27 @@ __device__ inline void pair_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-// inclusive prefix sum over the 16 lanes of a pair
+// inclusive prefix sum over the G lanes of a pair
+template <int G>
 __device__ inline uint32_t pair_scan(uint32_t v, int l) {
 #pragma unroll
-  for (int o = 1; o < kPairLanes; o <<= 1) {
-    const uint32_t t = __shfl_up(v, o, kPairLanes);
+  for (int o = 1; o < G; o <<= 1) {
+    const uint32_t t = __shfl_up(v, o, G);
     if (l >= o) v += t;
   }
   return v;
 }
+template <int G>
 __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nshapes, const uint32_t* __restrict__ gslot,
                                                           uint32_t* __restrict__ nown, uint32_t* __restrict__ fcount,
                                                           uint32_t* __restrict__ tmp, uint32_t* __restrict__ pool,
                                                           uint32_t pool_cap, uint32_t* __restrict__ fpool) {
+  constexpr int kEnumPairs = kEnumBlock / G, HL = G / 2;
   __shared__ ShapeIdx tab[XDEM_MAX_SHAPES];
-  __shared__ V3 verts[kEnumPairs][2][XDEM_MAX_SHAPE_VERTICES];
-  __shared__ FaceFrame frames[kEnumPairs][kPairLanes];
+  __shared__ V3 verts[kEnumPairs][2][HL];
+  __shared__ FaceFrame frames[kEnumPairs][G];
   // sixteen lanes per shape: edge l and, in lanes 0-7, face l (unused entries stay unread)
-  for (int k = (int)threadIdx.x / kPairLanes; k < nshapes; k += kEnumPairs) {
+  for (int k = (int)threadIdx.x / kPairLanes; k < nshapes; k += kEnumBlock / kPairLanes) {
     const xdem_shape& sh = a.shapes[k];
     ShapeIdx& t = tab[k];
     const int q = (int)threadIdx.x & (kPairLanes - 1);
@@ -618,9 +622,9 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
     }
   }
   __syncthreads();
-  const int l = (int)threadIdx.x & (kPairLanes - 1), pr = (int)threadIdx.x / kPairLanes;
-  const bool own = l < 8;  // the lane's vertex is the owner's
-  const int vi = l & 7;
+  const int l = (int)threadIdx.x & (G - 1), pr = (int)threadIdx.x / G;
+  const bool own = l < HL;  // the lane's vertex is the owner's
+  const int vi = l & (HL - 1);
   const double rv = a.rv;
   const int64_t total = (int64_t)nown[3];
   for (int64_t t = (int64_t)blockIdx.x * kEnumPairs + pr; t < total; t += (int64_t)gridDim.x * kEnumPairs) {
@@ -661,7 +665,7 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
     const V3s vo = own ? vb : va;
     // frames of the other body's faces, for the pair's lanes of this side (none without a gated vertex)
     const uint64_t gates = __ballot(gate);
-    const uint32_t side = (uint32_t)(gates >> (((int)threadIdx.x & 63) & ~7)) & 0xffu;
+    const uint32_t side = (uint32_t)(gates >> (((int)threadIdx.x & 63) & ~(HL - 1))) & ((1u << HL) - 1u);
     if (side && vi < (int)io.nf) frames[pr][l] = face_frame(vo, io.face[vi], (int)io.fsize[vi]);
     pair_fence();
     uint32_t vv = 0, ve = 0, vf = 0, ee = 0;
@@ -674,7 +678,7 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
         if (filter_ve(rv, v, rs, vo[io.edge[j][0]], vo[io.edge[j][1]], ro)) ve |= 1u << j;
       const double lim = rs + ro + rv;
       for (int j = 0; j < (int)io.nf; j++)
-        if (vf_frame(v, frames[pr][(l & 8) + j], lim)) vf |= 1u << j;
+        if (vf_frame(v, frames[pr][(l & HL) + j], lim)) vf |= 1u << j;
     }
     if (l < (int)ia.ne) {
       const V3 e0 = va[ia.edge[l][0]], e1 = va[ia.edge[l][1]];
@@ -698,9 +702,9 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
     }
     // positions: the owner's vertices, the edges, the partner's vertices
     const uint32_t nv_ = (uint32_t)(__popc(vv) + __popc(ve) + __popc(vf)), ne_ = (uint32_t)__popc(ee);
-    const uint32_t sv = pair_scan(nv_, l), se = pair_scan(ne_, l);
-    const uint32_t tv = __shfl(sv, 7, kPairLanes), te = __shfl(se, kPairLanes - 1, kPairLanes);
-    const uint32_t nf = __shfl(sv, kPairLanes - 1, kPairLanes) + te;
+    const uint32_t sv = pair_scan<G>(nv_, l), se = pair_scan<G>(ne_, l);
+    const uint32_t tv = __shfl(sv, HL - 1, G), te = __shfl(se, G - 1, G);
+    const uint32_t nf = __shfl(sv, G - 1, G) + te;
     uint32_t pb = ~0u;
     if (l == 0) {
       fcount[sl] = nf;
@@ -712,7 +716,7 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
         fpool[sl] = pb;
       }
     }
-    pb = __shfl(pb, 0, kPairLanes);
+    pb = __shfl(pb, 0, G);
     uint32_t* out = tmp + (int64_t)sl * kFeatPerSlot;
     uint32_t at = sv - nv_ + (own ? 0u : te);
     auto put = [&](uint32_t w) {
@@ -726,6 +730,19 @@ __global__ __launch_bounds__(kEnumBlock) void k_feat_enum(PolyNbhArgs a, int nsh
     at = tv + se - ne_;
     for (; ee; ee &= ee - 1u) put(feat_word(3, 0, l, __ffs(ee) - 1));
   }
+}
+
+// Lanes per pair of k_feat_enum: enough for the largest shape present (types: bit per type), one per vertex and face of
+// each body and one per edge. With sixteen for every shape most lanes of a smaller one idle, and its rebuild was slower
+// than with one thread per pair (ms per rebuild at 200k: one thread, sixteen lanes, this rule; tetrahedra 1.07, 1.31,
+// 0.95 with eight lanes; square plates 0.67, 0.54, 0.52 with eight; rods 0.49, 0.46, 0.46 with four; spheres 0.78, 0.95,
+// 0.79 with two). A cube or an octahedron among the particles takes sixteen.
+inline int pair_lanes(const xdem_shape* shapes, int n, uint32_t types) {
+  int lanes = 2;
+  for (int k = 0; k < n; k++)
+    if ((types >> k) & 1u)
+      while (2 * shapes[k].nv > lanes || 2 * shapes[k].nf > lanes || shapes[k].ne > lanes) lanes *= 2;
+  return lanes;
 }
 
 // One thread per pair of k_feat_enum: its feature words copied to their place in the list (slot order, from the
@@ -1212,9 +1229,16 @@ int poly_nbh(xdem_ctx* c, double rcut_inc) {
                        c->stream, L, c->oslot, c->d_nown);
     // about half of the slots are owner slots (both, for periodic images); blocks past their number return at once
     hipLaunchKernelGGL(k_pair_gate, gsl, bsl, 0, c->stream, a, c->oslot, c->d_nown, c->gslot);
-    const int64_t eblk = std::min<int64_t>(grid_blocks(std::max<int64_t>(L.slots, 1), kEnumPairs), kEnumBlocks);
-    hipLaunchKernelGGL(k_feat_enum, dim3((uint32_t)eblk), dim3(kEnumBlock), 0, c->stream, a, c->nshapes, c->gslot,
-                       c->d_nown, P.fcount, c->feat_tmp, c->feat_pool, (uint32_t)c->cap_feat_pool, c->feat_fpool);
+    const int lanes = pair_lanes(c->shapes, c->nshapes, c->type_mask);
+    const int64_t eblk = std::min<int64_t>(grid_blocks(std::max<int64_t>(L.slots, 1), kEnumBlock / lanes), kEnumBlocks);
+#define ENUM(G)                                                                                                        \
+  hipLaunchKernelGGL(k_feat_enum<G>, dim3((uint32_t)eblk), dim3(kEnumBlock), 0, c->stream, a, c->nshapes, c->gslot,     \
+                     c->d_nown, P.fcount, c->feat_tmp, c->feat_pool, (uint32_t)c->cap_feat_pool, c->feat_fpool)
+    if (lanes == 16) ENUM(16);
+    else if (lanes == 8) ENUM(8);
+    else if (lanes == 4) ENUM(4);
+    else ENUM(2);
+#undef ENUM
     if ((rc = scan_u64_from_u32(c, P.fcount, P.start, L.slots, 1u))) return rc;
   }
   uint64_t nf = 0;

@@ -412,6 +412,7 @@ struct xdem_ctx {
   bool cells_valid = false;     // cell_start matches the current positions and order
   bool hist_ready = false;      // history of the current list has been carried over (nbh_sphere)
   uint32_t max_type = 0;        // largest particle type of the last upload
+  uint32_t type_mask = 1;       // bit t: a particle of the last upload has type t (types of 31 and more: bit 31)
   bool ids_dense = false;       // the uploaded ids are a permutation of 0..n-1
   uint64_t nl_epoch = 0;        // number of neighbour builds so far
   uint64_t pl_epoch = ~0ull;    // neighbour build the feature lists were made from

@@ -398,6 +398,42 @@ def test_feature_enumeration_of_mixed_shapes(gpu_ok, n):
         assert {0, 1, 2, 3} <= set(gk[:, 2]) and set(gk[gk[:, 2] > 0, 3]) == {0, 1}
 
 
+@pytest.mark.parametrize("n", [7, 1203])
+@pytest.mark.parametrize("kinds", [("ball",), ("rod",), ("rod", "ball"), ("tetra",), ("plate", "rod"), ("tetra", "ball")])
+def test_feature_enumeration_of_small_shapes(gpu_ok, kinds, n):
+    """Two, four and eight lanes per pair: particles of shapes without cubes and octahedra (registered with them, which
+    does not count), whose vertices, edges and faces fill the lanes or leave some idle: the feature lists equal the
+    oracle's, word for word and in order."""
+    defs = {k: shp.ShapeDef(k) for k in ("rod", "ball", "tetra", "plate")}
+    defs["rod"].vertices, defs["rod"].edges = [(-0.6, 0.0, 0.0), (0.6, 0.0, 0.0)], [(0, 1)]
+    defs["ball"].vertices = [(0.0, 0.0, 0.0)]
+    defs["tetra"].vertices = [(0.5, 0.5, 0.5), (-0.5, -0.5, 0.5), (-0.5, 0.5, -0.5), (0.5, -0.5, -0.5)]
+    defs["tetra"].edges = [(0, 1), (0, 2), (0, 3), (1, 2), (1, 3), (2, 3)]
+    defs["tetra"].faces = [(0, 1, 2), (0, 3, 1), (0, 2, 3), (1, 3, 2)]
+    defs["plate"].vertices = [(0.5, 0.5, 0.0), (-0.5, 0.5, 0.0), (-0.5, -0.5, 0.0), (0.5, -0.5, 0.0)]
+    defs["plate"].edges, defs["plate"].faces = [(0, 1), (1, 2), (2, 3), (3, 0)], [(0, 1, 2, 3)]
+    for k, d in defs.items():
+        d.radius, d.volume, d.inertia_on_mass = 0.4 if k == "ball" else 0.05, 0.2, (0.1, 0.1, 0.1)
+    w = inputs.polyhedra(density=2500.0, n=n, spacing=0.85 if kinds == ("ball",) else 1.0, jitter=0.05, seed=n, dt=2e-4,
+                         z0=0.8, periodic=(n > 500, n > 500, False))
+    w.shapes = list(w.shapes) + [defs[k].to_record() for k in kinds]
+    w.particles["type"] = (2 + np.arange(n) * 7 // 3 % len(kinds)).astype(np.uint32)
+    o = oracle_for(w)
+    o.rebuild_poly(w.rcut_inc)
+    s = PolySim(w)
+    s.rebuild()
+    gk, gf = feature_table(*s.ctx.poly_interactions())
+    ok, of = feature_table(*o.poly_interactions())
+    assert np.array_equal(gk, ok) and np.array_equal(gf, of)
+    if n > 500:
+        types = set(gk[:, 2])
+        assert 0 in types
+        if "rod" in kinds or "tetra" in kinds:
+            assert {1, 3} <= types
+        if "tetra" in kinds:
+            assert 2 in types
+
+
 @pytest.mark.parametrize("n", [41, 1203])
 def test_histories_carried_over_rebuilds(gpu_ok, n):
     """Histories found again by feature: after several rebuilds with pairs in contact the lists and friction histories
