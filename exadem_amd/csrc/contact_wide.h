@@ -195,11 +195,7 @@ __global__ __launch_bounds__(256) void k_force_wide(typename P::Args a) {
     }
   }
   if (!lin && !rot) return;
-  if (a.mt.ncand && a.mt.wcnt[xi >> 6] != 0u) {
-    const uint2 mi = a.mt.idx[xi];
-    const double* t = a.mt.terms + (int64_t)mi.x * 6 + c0;
-    for (uint32_t u = 0; u < mi.y; u++) S = S + V3{t[6 * u], t[6 * u + 1], t[6 * u + 2]};
-  }
+  if (a.mt.ncand && a.mt.wcnt[xi >> 6] != 0u) mesh_add_half(a.mt, a.mt.idx[xi], c0, S);
   d4 ra{}, rb{};
   V3 ex{0.0, 0.0, 0.0};
   if (FUSED) {  // position and velocity halves of the record, or spin and orientation

@@ -246,5 +246,24 @@ __device__ inline void mesh_add_at(const MeshTerms& t, uint2 mi, V3& F, V3& M) {
     }
   }
 }
+// The force (c0 = 0) or the moment terms (c0 = 3) alone, in the same order, with the loads of four candidates in flight
+// (the several-lanes pass, in which a thread of its own sums each of the two). One load after the other made a step of
+// 20,000 spheres on a mesh of spacing 0.5 (up to about 20 candidates per sphere on it) 23.1 us, slower than the one-lane pass
+// (22.4); now 19.8. (The gather of polyhedra keeps the plain loop: with the batch its rolling form spills more registers,
+// 218 -> 222 us at 200,000.)
+__device__ inline void mesh_add_half(const MeshTerms& t, uint2 mi, int c0, V3& S) {
+  const double* p = t.terms + (int64_t)mi.x * 6 + c0;
+  for (uint32_t k0 = 0; k0 < mi.y; k0 += 4) {
+    V3 r[4];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++) {
+      const uint32_t k = k0 + q < mi.y ? k0 + q : k0;  // past the end: the batch's first again, not added
+      r[q] = V3{p[6 * k], p[6 * k + 1], p[6 * k + 2]};
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++)
+      if (k0 + q < mi.y) S = S + r[q];
+  }
+}
 
 }  // namespace xdem

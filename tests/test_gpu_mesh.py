@@ -11,7 +11,7 @@ the mesh history over) and of the engine within 1e-10 after 60 steps.
 import numpy as np
 import pytest
 
-from exadem_amd import native
+from exadem_amd import native, stl
 from exadem_amd.sim import SphereSim, scheme
 import pyoracle as po
 
@@ -95,6 +95,32 @@ def test_mesh_matches_oracle(gpu_ok, rm):
     assert np.array_equal(kg, ko)
     assert float(np.max(np.abs(fg - fo))) <= 1e-12 * max(1e-30, float(np.max(np.abs(fo))))
     print(f"rm={rm}: {w.n} spheres, active mesh contacts at the first pass {active}")
+
+
+@pytest.mark.parametrize("kr", [0.0, 2e3])
+def test_many_candidates_match_oracle(gpu_ok, kr):
+    """A mesh much finer than the spheres: the terms of up to several tens of candidates per sphere are added in
+    candidate order (batches of four, the last one partial), with and without a rolling stiffness: forces, state and
+    histories equal the oracle's bit for bit."""
+    w = mc.workload("tray", mc.tray_bed())
+    w.cp = w.cpd = native.contact_params(kn=1e5, mu=0.3, damp_rate=0.9, kr=kr)
+    v, e, f = stl.build_shape(mc.tray_triangles(n=64, h=0.3125, apex=0.0))
+    m = {"mesh_id": 6, "vertices": v, "edges": e, "faces": f, "minkowski": 0.0}
+    sch = scheme(w)
+    o = oracle_for(w, m)
+    o.first_iteration(sch)
+    o.run_steps(sch, 20)
+    s = SphereSim(w, mesh=dict(m, max_candidates=96))
+    s.first_iteration()
+    s.run(20, poll=7)
+    g, q = by_id(s.ctx.download()), by_id(o.particles())
+    for k in ("rx", "ry", "rz", "vx", "vy", "vz", "vrotx", "vroty", "vrotz", "fx", "fy", "fz", "momx", "momy", "momz"):
+        assert np.array_equal(g[k], q[k]), k
+    kg, fg = mesh_table(*s.ctx.mesh_interactions()[:4])
+    ko, fo = mesh_table(*o.mesh_interactions()[:4])
+    assert np.array_equal(kg, ko) and np.array_equal(fg, fo)
+    count = np.bincount(kg[:, 0])
+    assert count.max() > 20 and len(set(count[count > 0] % 4)) == 4
 
 
 def test_mesh_errors(gpu_ok):
