@@ -407,7 +407,7 @@ int launch_step(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd, 
   a.core_out = c->core_alt;
   a.kdt_2 = dt * 0.5;
   a.thr2 = thr2;
-  if (const int lanes = wide_lanes(a.n, c->nl_max_rows); lanes > 1) {
+  if (const int lanes = wide_lanes(a.n, a.nl.slots, c->nl_max_rows, false, c->kr_used); lanes > 1) {
     if (c->kr_used) launch_wide<WideFp64<true>>(c, a, lanes, true, true, true);
     else launch_wide<WideFp64<false>>(c, a, lanes, true, true, true);
     return finish_step(c, a.trig_out, input);
@@ -481,7 +481,7 @@ int launch_force(xdem_ctx* c, const ContactParams& cp, const ContactParams& cpd,
     }
   }
   if (meshed && (rc = launch_mesh_pass(c, cpd, dt, guarded, c->trig_slot, mstate, &a.mt))) return rc;
-  const int lanes = wide_lanes(a.n, c->nl_max_rows);
+  const int lanes = wide_lanes(a.n, a.nl.slots, c->nl_max_rows, false, c->kr_used);
   if (lanes > 1 && !c->record_cs && (fused || !guarded)) {
     if (c->kr_used) launch_wide<WideFp64<true>>(c, a, lanes, fused, false, guarded);
     else launch_wide<WideFp64<false>>(c, a, lanes, fused, false, guarded);

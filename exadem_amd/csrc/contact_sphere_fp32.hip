@@ -448,7 +448,7 @@ int launch_force_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams&
   a.step_tag = step_tag;
   a.trig_in = c->trig_slot;
   const bool kr = c->kr_used;
-  const int lanes = wide_lanes(a.n, c->nl_max_rows);
+  const int lanes = wide_lanes(a.n, a.nl.slots, c->nl_max_rows, true, c->kr_used);
   if (lanes > 1 && (fused || !guarded)) {
     if (kr) launch_wide<WideFp32<true>>(c, a, lanes, fused, false, guarded);
     else launch_wide<WideFp32<false>>(c, a, lanes, fused, false, guarded);
@@ -496,7 +496,7 @@ int launch_step_fp32(xdem_ctx* c, const ContactParams& cp, const ContactParams& 
   a.core_out = c->core_alt;
   a.kdt_2 = dt * 0.5;
   a.thr2 = thr2;
-  if (const int lanes = wide_lanes(a.n, c->nl_max_rows); lanes > 1) {
+  if (const int lanes = wide_lanes(a.n, a.nl.slots, c->nl_max_rows, true, c->kr_used); lanes > 1) {
     if (c->kr_used) launch_wide<WideFp32<true>>(c, a, lanes, true, true, true);
     else launch_wide<WideFp32<false>>(c, a, lanes, true, true, true);
     return finish_step(c, a.trig_out, input);

@@ -3,8 +3,8 @@
 //
 // With one lane per particle a pass lasts as long as the longest chain of one lane: its list entries one after the
 // other (6 to 14 contacts of FP64 detection and law, each behind a gather), the walls, the mesh terms, the
-// integration. Up to some tens of thousands of particles that chain, not bandwidth, is the time of a step (14 to
-// 15 us at 1k to 30k spheres). Here L lanes share a particle: each evaluates one list entry of a round of L, writes
+// integration. Up to some tens of thousands of particles that chain, not bandwidth, is the time of a step (15 to
+// 19 us at 1k to 36k spheres). Here L lanes share a particle: each evaluates one list entry of a round of L, writes
 // the six terms it adds to the particle to LDS, and two threads per particle (force, moment) add them in list order, so
 // the sums and their order, and with them every bit of the result, are those of the one-lane pass. Lanes without a
 // contact write -0.0, which adds nothing to any value. The walls are a round of their own (one lane per wall); the
@@ -241,20 +241,37 @@ __global__ __launch_bounds__(256) void k_force_wide(typename P::Args a) {
   }
 }
 
-// Lanes per particle of a pass over n spheres whose longest list has `rows` entries; 1: the one-lane kernels. Per step of
-// the engine (us, FP64; one lane / four / eight; a walled lattice with 6 entries per sphere, then a periodic packing
-// with up to 14):
-//   1,000: 16.8 / 11.4 / 8.6              5,000: 16.4 / 11.4 / 8.8, 21.6 / 10.7 / 8.9
-//   20,000: 16.3 / 13.5 / 11.6, 21.9 / 14.2 / 13.1    36,000: 16.9 / 15.7 / 15.7, 23.1 / 17.3 / 15.4
-//   40,000: 17.5 / 16.2 / 16.8, 22.5 / 17.3 / 17.2    60,000: 18.4 / 19.7 / 20.4, 23.8 / 20.8 / 22.2
-//   80,000: 22.8 / 25.4 / 25.8, 30.4 / 25.9 / 27.6
-// Beyond, the shared lanes' extra work (records read by every lane, sums through LDS) costs more than the shorter chain
-// saves; with short lists that point comes earlier. Two lanes per particle were never the best of the four.
-constexpr int64_t kWide8Max = 36000, kWide4Max = 64000, kWide4MaxShort = 45000;
-constexpr int kWideShortRows = 8;
-inline int wide_lanes(int64_t n, int rows) {
+// Lanes per particle of a pass over n spheres whose list has `slots` slots (a group of 64 particles has the rows of its
+// longest list, so slots / n is the rows of an average wavefront) and whose longest row is `longest`; 1: the one-lane
+// kernels. Per step of the engine, without rebuilds (us; one lane / four / eight):
+//                     walled lattice (5.9 rows)    periodic packing (7.1 rows)    wide size distribution (8.1 rows)
+//   FP64    5,000:    14.8 / 10.7 /  8.3           16.3 /  9.6 /  7.9
+//          20,000:    14.7 / 13.0 / 11.3           17.2 / 12.6 / 12.1             22.8 / 14.4 / 12.3
+//          36,000:    15.4 / 15.2 / 15.3           18.4 / 15.8 / 14.4             22.1 / 17.0 / 14.9
+//          45,000:    15.9 / 16.0 / 17.5           19.0 / 16.6 / 17.7             23.2 / 18.1 / 18.6
+//          49,000:    16.0 / 16.4 / 18.0           19.0 / 16.6 / 19.2             22.9 / 18.1 / 20.4
+//          52,000:    16.4 / 18.5 / 18.7           18.9 / 18.9 / 19.3             24.3 / 21.6 / 20.1
+//          64,000:    17.2 / 18.7 / 21.2           19.6 / 19.5 / 21.6             24.4 / 21.8 / 22.8
+//          80,000:    22.1 / 24.5 / 24.8           24.9 / 25.0 / 25.6
+//   FP32   20,000:    15.2 / 12.7 / 11.1           17.6 / 12.0 / 11.3             24.1 / 13.7 / 12.3
+//          49,000:    16.3 / 15.6 / 17.7           19.2 / 15.1 / 18.4             23.5 / 16.8 / 20.0
+//          52,000:    16.8 / 17.4 / 18.2           19.1 / 16.9 / 18.6             25.0 / 19.5 / 19.9
+//          64,000:    17.5 / 17.4 / 20.8           19.5 / 17.6 / 21.3             24.5 / 19.8 / 22.3
+//          80,000:    20.9 / 23.0 / 24.5           23.4 / 22.7 / 24.8
+// The four-lane times step up where the blocks of 64 particles pass three and four per CU. One crowded sphere in the
+// walled lattice (a row of 12) delays one wavefront of the one-lane pass: 49,000: 16.8 / 16.4, 60,000: 17.4 / 18.9 in
+// FP64 and 17.7 / 17.8 in FP32; so the longest row alone decides only up to three blocks per CU in FP64 and four in FP32.
+// With a rolling stiffness (more registers) four blocks are never worth it in FP64 nor, with short lists, in FP32: 64,000
+// spheres, walled lattice 22.4 / 29.4 and 23.1 / 26.2, periodic 25.4 / 26.5 and 24.7 / 23.6.
+constexpr int64_t kWide8Max = 36000, kWideShort = 45000;
+constexpr int64_t kWide3 = 3 * 256 * 64, kWide4 = 4 * 256 * 64;  // spheres at three, four blocks of 64 per CU
+inline int wide_lanes(int64_t n, int64_t slots, int longest, bool fp32, bool kr) {
   if (n <= kWide8Max) return 8;
-  return n <= (rows > kWideShortRows ? kWide4Max : kWide4MaxShort) ? 4 : 1;
+  const bool mid = 2 * slots >= 13 * n, big = 2 * slots >= 15 * n;  // 6.5 and 7.5 rows
+  int64_t most;
+  if (fp32) most = mid || (longest > 8 && !kr) ? kWide4 : kWide3;
+  else most = big && !kr ? kWide4 : mid || longest > 8 ? kWide3 : kWideShort;
+  return n <= most ? 4 : 1;
 }
 
 template <class P>
