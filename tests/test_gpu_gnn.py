@@ -165,6 +165,46 @@ def test_backward_sizes_match_oracle(gpu_ok, n):
     gnn.close()
 
 
+def test_backward_of_several_stages_matches_oracle(gpu_ok):
+    """Gradients at a size where the training kernels' loops run more than once: 20,011 spheres are three stages of 64
+    rows in a weight gradient's block (the last one partial) and a second group of 32 particles in some blocks of the
+    message backward.
+
+    The residual keeps its sign (0.5 to 1.5 of the outputs' scale). The two pipelines' outputs differ by at most 1e-2 of
+    that scale (the forward bar), and by about the same at similar particles: against a residual of zero mean, whose
+    gradient over n particles falls like 1 / sqrt(n), that difference stays, and 2.6e-2 was seen at this n with a
+    deviation of 0.5 (the same to four digits with a per-edge scalar backward); against this one it is 1e-2 of the
+    gradient, and the bfloat16 bar of the backward itself, 1e-2 (2^-9 per stored value and the gates it flips), is added."""
+    w = periodic_pack(n=20011, sigma_v=0.3)
+    rng = np.random.default_rng(9)
+    for k in ("vrotx", "vroty", "vrotz"):
+        w.particles[k] = rng.normal(0, 0.2, w.n)
+    sim = SphereSim(w)
+    sim.first_iteration()
+    flat = _params(17)
+    gnn = native.Gnn(sim.ctx, r0=0.4, v0=0.1, a0=1.0, m0=4000.0, ov_scale=50.0, substeps=10, train=True)
+    gnn.set_params(flat)
+    out = gnn.forward()
+    sign = np.array([1.0, -1.0, 1.0, 1.0, -1.0, 1.0])
+    target = (out + float(np.max(np.abs(out))) * sign * rng.uniform(0.5, 1.5, (w.n, 1))).astype(np.float32)
+    gnn.set_target(target)
+    loss = gnn.backward()
+    grads = gnn.get_grads()
+    src, dst, e, x = gnn.dump_graph()
+    onet = G.Net(flat.astype(np.float64), exact=False)
+    o_out, cache = onet.forward(x, src.astype(np.int64), dst.astype(np.int64), e)
+    assert float(np.max(np.abs(out - o_out))) <= 1e-2 * float(np.max(np.abs(o_out)))
+    assert loss == pytest.approx(onet.loss(o_out, target), rel=2e-2)
+    og = onet.backward(cache, target)
+    off = 0
+    for name, shape in G.param_layout():
+        k = int(np.prod(shape))
+        a, b = grads[off:off + k].astype(np.float64), np.asarray(og[name], np.float64).ravel()
+        off += k
+        assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b), (name, np.linalg.norm(a - b) / np.linalg.norm(b))
+    gnn.close()
+
+
 def test_training_lowers_loss_and_beats_free_flight(gpu_ok):
     """The library's training loop on 16 packings of 4000 spheres (25 windows of 10 DEM steps each);
     then, on windows of a packing it has not seen, the network's acceleration error against the DEM
