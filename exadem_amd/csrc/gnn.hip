@@ -27,10 +27,15 @@ constexpr int H = XDEM_GNN_HIDDEN, L = XDEM_GNN_LAYERS, FN = 8, FE = 16, FO = 6,
 constexpr float kMsgScale = 0.125f;
 constexpr int kRedBlocks = 512;  // blocks of the grid-stride reduction kernels (partial sums)
 constexpr int kWgChunks = 128;   // most row chunks of a weight gradient
-// partial sums of one backward pass: per layer two weight gradients of H x 2H with a bias and the message
-// gradients, then the decoder (its outputs and the loss) and the encoder
-constexpr int64_t kPartialFloats = (int64_t)L * (kWgChunks * (2 * H * H2 + H) + kRedBlocks * H * (FE + 1)) +
-                                   (int64_t)kRedBlocks * (FO * H + FO + 1 + H * (FN + 1));
+constexpr int kWgRows = 64;      // rows of a stage of a weight gradient, the fewest of a chunk
+// most partial sums of one backward pass over up to n particles: per layer two weight gradients of H x 2H with a bias
+// and the message gradients, then the decoder (its outputs and the loss) and the encoder. 118 MB from 8,192 particles
+// on, 16 MB at 1,000.
+inline int64_t partial_floats(int64_t n) {
+  const int64_t chunks = std::min<int64_t>(kWgChunks, (n + kWgRows - 1) / kWgRows);
+  const int64_t msg = std::min<int64_t>(kRedBlocks, (n + 31) / 32), rows = std::min<int64_t>(kRedBlocks, (n + 3) / 4);
+  return L * (chunks * (2 * H * H2 + H) + msg * H * (FE + 1)) + rows * (FO * H + FO + 1 + H * (FN + 1));
+}
 
 struct Off {
   int64_t W_in, b_in, W_AB[L], W_E[L], b_E[L], W_U[L], b_U[L], W_out, b_out, total;
@@ -402,7 +407,7 @@ struct WgradArgs {
   float* partial;  // [gridDim.x][mg * K]
   float* part_b;   // [gridDim.x][128] (null: no bias gradient)
 };
-constexpr int kWgRows = 64, kWgStride = kWgRows + 8;
+constexpr int kWgStride = kWgRows + 8;
 __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
   __shared__ uint16_t tile[256 * kWgStride];
   const WgradHalf hf = a.h[blockIdx.y];
@@ -1264,7 +1269,7 @@ struct xdem_gnn {
   uint16_t* dpq = nullptr;
   uint32_t* mirror = nullptr;
   uint32_t* gate = nullptr;  // gates of the messages' backward pass (MsgArgs::gate)
-  float* partial = nullptr;  // partial sums of a backward pass (training; sized once, never reallocated)
+  float* partial = nullptr;  // partial sums of a backward pass (training; sized with the particles)
   int64_t cap_partial = 0;
   double* snap = nullptr;
   double* xs = nullptr;
@@ -1286,6 +1291,18 @@ int galloc(xdem_ctx* c, T** p, int64_t count) {
   return XDEM_OK;
 }
 
+// capacity of the per-particle buffers for n particles
+inline int64_t cap_of(int64_t n) { return (int64_t)(n * 1.1) + 256; }
+int ensure_partial(xdem_gnn* G, int64_t n) {
+  const int64_t floats = partial_floats(n);
+  if (floats <= G->cap_partial) return XDEM_OK;
+  G->cap_partial = 0;
+  int rc = galloc(G->c, &G->partial, floats);
+  if (rc) return rc;
+  G->cap_partial = floats;
+  return XDEM_OK;
+}
+
 int ensure_buffers(xdem_gnn* G) {
   xdem_ctx* c = G->c;
   const int64_t n = c->n;
@@ -1298,7 +1315,7 @@ int ensure_buffers(xdem_gnn* G) {
     G->cap_slots = cap;
   }
   if (n > G->cap_n) {
-    const int64_t cap = (int64_t)(n * 1.1) + 256;
+    const int64_t cap = cap_of(n);
     const int nh = G->cfg.train ? L + 1 : 2;
     const int nl_ = G->cfg.train ? L : 1;
     if ((rc = galloc(c, &G->x, cap * FN))) return rc;
@@ -1313,7 +1330,7 @@ int ensure_buffers(xdem_gnn* G) {
     if (G->cfg.train) {
       if ((rc = galloc(c, &G->target, cap * FO)) || (rc = galloc(c, &G->dh, cap * H)) ||
           (rc = galloc(c, &G->dm, cap * H)) || (rc = galloc(c, &G->du, cap * H)) ||
-          (rc = galloc(c, &G->dpq, cap * H2)) || (rc = galloc(c, &G->snap, cap * 6)))
+          (rc = galloc(c, &G->dpq, cap * H2)) || (rc = galloc(c, &G->snap, cap * 6)) || (rc = ensure_partial(G, cap)))
         return rc;
     }
     if ((rc = galloc(c, &G->xs, cap * 3)) || (rc = galloc(c, &G->xf, cap * 3))) return rc;
@@ -1542,11 +1559,10 @@ extern "C" int xdem_gnn_create(xdem_ctx* c, const xdem_gnn_config* cfg, xdem_gnn
   if ((rc = galloc(c, &G->p, np)) || (rc = galloc(c, &G->g, np + 1)) || (rc = galloc(c, &G->m1, np)) ||
       (rc = galloc(c, &G->m2, np)) || (rc = galloc(c, &G->wbf, np)) || (rc = galloc(c, &G->wr, np)) ||
       (rc = galloc(c, &G->wT, (int64_t)L * 2 * H * H2)) || (rc = galloc(c, &G->dpart, 4 * 65536)) ||
-      (cfg->train && (rc = galloc(c, &G->partial, kPartialFloats)))) {
+      (cfg->train && (rc = ensure_partial(G, cap_of(c->n))))) {
     delete G;
     return rc;
   }
-  G->cap_partial = cfg->train ? kPartialFloats : 0;
   XDEM_HIP(c, hipMemsetAsync(G->p, 0, sizeof(float) * np, c->stream));
   XDEM_HIP(c, hipMemsetAsync(G->g, 0, sizeof(float) * np, c->stream));
   XDEM_HIP(c, hipMemsetAsync(G->m1, 0, sizeof(float) * np, c->stream));

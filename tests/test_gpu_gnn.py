@@ -205,6 +205,38 @@ def test_backward_of_several_stages_matches_oracle(gpu_ok):
     gnn.close()
 
 
+def test_memory_of_a_small_training_network(gpu_ok):
+    """A training network takes device memory for its particles, not for the most that its reductions ever need: under
+    40 MB at 1,000 spheres (16 MB of partial sums, 6 MB of activations, 5 MB of parameters and the graph), and a backward
+    pass after the particles have become many more still has room for its partial sums."""
+    import torch
+    free = lambda: torch.cuda.mem_get_info(0)[0]
+    small, large = SphereSim(periodic_pack(n=1000, sigma_v=0.3)), periodic_pack(n=9000, sigma_v=0.3)
+    small.first_iteration()
+    before = free()
+    gnn = native.Gnn(small.ctx, r0=0.4, v0=0.1, a0=1.0, m0=4000.0, ov_scale=50.0, substeps=10, train=True)
+    gnn.set_params(_params(3))
+    out = gnn.forward()
+    gnn.set_target(out + 1.0)
+    assert gnn.backward() == pytest.approx(1.0, rel=1e-3)
+    assert before - free() < 40e6
+    small.ctx.set_domain(large.domain)
+    small.ctx.upload(large.particles)
+    small.rebuild()
+    out = gnn.forward()
+    gnn.set_target(out + 1.0)
+    assert gnn.backward() == pytest.approx(1.0, rel=1e-3)
+    ref = SphereSim(large)
+    ref.first_iteration()
+    other = native.Gnn(ref.ctx, r0=0.4, v0=0.1, a0=1.0, m0=4000.0, ov_scale=50.0, substeps=10, train=True)
+    other.set_params(_params(3))
+    other.set_target(other.forward() + 1.0)
+    other.backward()
+    assert np.array_equal(gnn.get_grads(), other.get_grads())
+    gnn.close()
+    other.close()
+
+
 def test_training_lowers_loss_and_beats_free_flight(gpu_ok):
     """The library's training loop on 16 packings of 4000 spheres (25 windows of 10 DEM steps each);
     then, on windows of a packing it has not seen, the network's acceleration error against the DEM
