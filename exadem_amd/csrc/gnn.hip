@@ -714,7 +714,8 @@ __device__ inline void bwd_load(const MsgArgs& a, uint64_t sl, bool ok, uint32_t
   }
 }
 // v_writelane_b32: `old` with its value in one lane replaced by the uniform `val` (no clang builtin; the compiler's
-// own intrinsic, so that it keeps the instruction's hazards)
+// own intrinsic, so that it keeps the instruction's hazards). With a compiler that does not know the intrinsic by this
+// name the function stays undefined and the device link fails.
 __device__ int amdgcn_writelane(int val, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 __device__ inline uint32_t write_lane(uint32_t old, uint32_t val, int lane) {
   return (uint32_t)amdgcn_writelane((int)val, lane, (int)old);

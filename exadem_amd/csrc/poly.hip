@@ -553,9 +553,10 @@ __global__ __launch_bounds__(256) void k_pair_gate(PolyNbhArgs a, const uint32_t
 // frames and the shapes' index tables are shared through LDS. A lane's hits are bit masks; prefix sums over the pair's
 // lanes put the words into the order of for_each_feature. The count and up to kFeatPerSlot feature words go to the slot's
 // region of tmp.
-// FP64 arithmetic bounds it (144 edge pairs, up to 96 vertex-edge and 14 face tests per cube pair). A lattice of spacing
-// 1.35 to 1.4: 163 us at 20k polyhedra, 1.37 ms at 200k (175 us and 1.49 ms with filter_ee on every edge pair); one
-// thread per pair (164 registers, three wavefronts per SIMD, one long chain per thread) took 360 us and 1.88 ms.
+// FP64 arithmetic bounds it (a cube pair: 144 edge pairs and, for vertices that pass their box gate, up to 192 vertex-edge
+// and 96 vertex-face tests against 12 face frames). A lattice of cubes and octahedra of spacing 1.35 to 1.4: 163 us at 20k
+// polyhedra, 1.34 ms at 200k (175 us and 1.49 ms with filter_ee on every edge pair); one thread per pair (164 registers,
+// three wavefronts per SIMD, one long chain per thread) took 360 us and 1.88 ms.
 constexpr int kFeatPerSlot = 24;
 // Features past kFeatPerSlot go to a chunk of kPoolChunk words claimed from a shared pool (counter nown[2], capacity
 // pool_cap); fpool[sl] = the chunk, or ~0u when the pool is exhausted or the pair has more than kFeatPerSlot + kPoolChunk
@@ -1657,8 +1658,8 @@ __global__ __launch_bounds__(128) void k_poly_feat(PolyForceArgs a) {
 // vertices of the new pose and test their displacement (flags[0] raised for the next step's pass).
 //
 // With one thread per particle, which walked its entries and their contacts one after the other, the pass lasted as long
-// as the longest such walk (57 us at 20k polyhedra in a dense moving bed), and the prolog with the vertices was a pass
-// of its own (31 us at 200k). Engine step: 64.8 -> 39.2 us at 20k moving, 94.0 -> 73.1 us at 200k at rest.
+// as the longest such walk, and the prolog with the vertices was a pass of its own (31 us at 200k). Step of the engine
+// between rebuilds, in a dense moving bed: 46.0 -> 20.4 us at 20k, 110 -> 86 us at 200k; at rest 93 -> 73 us at 200k.
 __device__ inline d4 rec_d4(const uint4* p) {  // LDS rows of records are 16-byte aligned
   d4 v;
   __builtin_memcpy(&v, p, sizeof(d4));
@@ -1942,10 +1943,11 @@ __global__ __launch_bounds__(256, 4) void k_poly_gather(PolyForceArgs a) {
   }
 }
 
-// Lanes per particle of the gather (us per step of the engine, eight / four / two lanes, a moving bed and at 200,000 the
-// bed at rest): 2,000: 30.3 / 32.1 / 39.5; 20,000: 39.2 / 39.5 / 45.1; 60,000: 72.0 / 66.5 / 71.7; 200,000: 84.0 / 73.1 /
-// 73.1. A block's life is its chain of dependent loads and barriers: while all blocks of 32 particles are resident at once
-// (four per CU at 118 registers, 256 CUs) the shortest chain wins, beyond that the fewest blocks.
+// Lanes per particle of the gather (us per step of the engine between rebuilds, eight / four lanes; a dense moving bed, and
+// the bed at rest): 2,000: 15.8 / 17.5, 12.9 / 13.9; 20,000: 20.4 / 21.1, 17.1 / 17.6; 32,000: 24.8 / 25.0, 20.6 / 20.3;
+// 40,000: 31.9 / 28.6, 26.9 / 23.5; 60,000: 38.6 / 34.2, 32.6 / 28.1; 200,000: 96.6 / 86.0, 83.9 / 73.4. A block's life is
+// its chain of dependent loads and barriers: while all blocks of 32 particles are resident at once (four per CU at 118
+// registers, 256 CUs) the shortest chain wins, beyond that the fewest blocks. (Two lanes were no better at 200,000.)
 constexpr int64_t kGather8Max = 4 * 256 * 32;
 inline int gather_lanes(int64_t n) { return n <= kGather8Max ? 8 : 4; }
 
